@@ -36,6 +36,7 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 constexpr int kMaxHeadDim = 1024;
 constexpr int kGenericMaxTopk = 12288;  // scores of one row stay in 64 KiB of LDS
+static_assert(sfa::kMlaGMaxTopk == kGenericMaxTopk, "these shapes take the top-k the generic kernel took");
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -140,10 +141,11 @@ struct FwdPlan {
 constexpr int kTargetWorkgroups = 512;  // 2 per CU on a 256-CU MI355X
 constexpr int kMaxSplits = 64;  // the combine kernel holds one split per lane of a wave
 
-// sort_room: the most workspace bytes the sorted index rows may take
-// (sfa_fwd_noalloc: what its static scratch leaves); rows that do not fit
-// are used in their own order.
-FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t sort_room = SIZE_MAX) {
+// room: the workspace bytes there are (sfa_fwd_noalloc: its static scratch).
+// Sorted index rows that do not fit are used in their own order; a kernel
+// that can walk any top-k in one item (fwd_partials_f32) is split no further
+// than its partials fit.
+FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SIZE_MAX) {
   FwdPlan pl{};
   sfa::Params p = to_params(a, pg);
   pl.mfma = mfma_layout_ok(a) && sfa::fwd_mfma_supported(p);
@@ -159,6 +161,11 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t sort_room
     } else if (items < kTargetWorkgroups / 2) {
       // decode-like: too few work items to fill the chip -> split the top-k set
       splits = (int)((kTargetWorkgroups / 2 + items - 1) / items);
+      // (the kernel for few heads: at least 4 tiles a split.  Measured at
+      // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 33.7 / 23.3 /
+      // 20.3 us, 64 splits 38.5 / 35.2 / 24.7 us: shorter splits load more Q
+      // and write more partial rows than the idle CUs repay)
+      if (sfa::fwd_partials_f32(p) && splits > (a->topk + 4 * nk - 1) / (4 * nk)) splits = (a->topk + 4 * nk - 1) / (4 * nk);
     }
     // each split must fit the staged index window and hold at least one tile
     const int min_splits = (a->topk + idx_cap - 1) / idx_cap;
@@ -167,6 +174,11 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t sort_room
     if (splits > max_splits) splits = max_splits;
     if (splits > kMaxSplits) splits = kMaxSplits;
     if (splits < 1) splits = 1;
+    const size_t rows = (size_t)a->B * a->Sq * a->Hq;
+    if (sfa::fwd_partials_f32(p) && room != SIZE_MAX) {
+      const size_t per_split = rows * (a->Dv + 1) * sizeof(float), fit = room < 512 ? 0 : (room - 512) / per_split;
+      if ((size_t)splits > fit) splits = fit > 1 ? (int)fit : 1;
+    }
     int len = (a->topk + splits - 1) / splits;
     len = (len + nk - 1) / nk * nk;
     splits = (a->topk + len - 1) / len;
@@ -178,7 +190,8 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t sort_room
   pl.num_splits = splits;
   if (splits > 1) {
     const size_t rows = (size_t)a->B * a->Sq * a->Hq;
-    pl.part_o_bytes = align_up((size_t)splits * rows * a->Dv * sizeof(__bf16), 256);
+    pl.part_o_bytes =
+        align_up((size_t)splits * rows * a->Dv * (sfa::fwd_partials_f32(p) ? sizeof(float) : sizeof(__bf16)), 256);
     pl.part_lse_bytes = align_up((size_t)splits * rows * sizeof(float), 256);
   }
   if (pl.mfma) {
@@ -191,7 +204,7 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t sort_room
       // logical keys), so a paged call walks the same slots as a contiguous one
       if (!(a->flags & SFA_FWD_IDX_SORTED) && sfa::idx_sort_supported(p)) {
         const size_t bytes = align_up((size_t)a->B * a->Sq * a->Hkv * a->topk * sizeof(int32_t), 256);
-        if (bytes + pl.sched_bytes <= sort_room) pl.sort_bytes = bytes;
+        if (bytes + pl.sched_bytes <= room) pl.sort_bytes = bytes;
       }
     }
   }
@@ -207,9 +220,9 @@ int check_generic_fwd(const sfa_fwd_args* a) {
 
 // The forward of sfa_fwd (pg == nullptr) and sfa_fwd_paged, after validation.
 int run_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, void* workspace, size_t workspace_bytes, void* stream,
-            size_t sort_room = SIZE_MAX) {
+            size_t room = SIZE_MAX) {
   hipStream_t s = (hipStream_t)stream;
-  const FwdPlan pl = plan_fwd(a, pg, sort_room);
+  const FwdPlan pl = plan_fwd(a, pg, room);
   sfa::Params p = to_params(a, pg);
   int rc;
   hipError_t e;
@@ -219,7 +232,10 @@ int run_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, void* workspace, size
     if (pl.workspace() > 0 && (workspace == nullptr || workspace_bytes < pl.workspace()))
       return fail(SFA_E_WORKSPACE, "sfa_fwd needs %zu workspace bytes (got %zu)", pl.workspace(), workspace_bytes);
     if (pl.num_splits > 1) {
-      p.part_o = (__bf16*)workspace;
+      if (sfa::fwd_partials_f32(p))
+        p.part_of = (float*)workspace;
+      else
+        p.part_o = (__bf16*)workspace;
       p.part_lse = (float*)((char*)workspace + pl.part_o_bytes);
     }
     if (pl.sched_bytes > 0) p.sched = (int*)((char*)workspace + pl.part_o_bytes + pl.part_lse_bytes);
@@ -235,7 +251,7 @@ int run_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, void* workspace, size
     e = sfa::launch_fwd_mfma(p, s);
     if (e != hipSuccess) return hip_fail(e, "sfa_fwd (mfma)");
     if (pl.num_splits > 1) {
-      e = sfa::launch_combine(p, a->dtype, s);
+      e = p.part_of ? sfa::launch_combine_f32(p, s) : sfa::launch_combine(p, a->dtype, s);
       if (e != hipSuccess) return hip_fail(e, "sfa_fwd (combine)");
     }
     return SFA_OK;

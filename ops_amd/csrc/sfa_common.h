@@ -46,6 +46,7 @@ struct Params {
   int num_splits;
   int split_len;      // slots per split (multiple of the key tile)
   __bf16* part_o;     // [num_splits][B*Sq*Hq][Dv] bf16, normalised by the split's own sum
+  float* part_of;     // the same in fp32 (fwd_partials_f32), instead of part_o
   float* part_lse;    // [num_splits][B*Sq*Hq], base-2 log-sum-exp of the split (-inf if empty)
   int* sched;         // persistent forward: 8 claim counters (one per XCD), zeroed before the launch
   // backward
@@ -347,6 +348,12 @@ bool fwd_mfma_persistent(const Params& p);  // needs Params::sched (8 ints of wo
 bool idx_sort_supported(const Params& p);
 hipError_t launch_idx_sort(const Params& p, int32_t* out, hipStream_t s);
 int fwd_mfma_head_groups(const Params& p);  // workgroups per (work item, split): head groups
+// MLA rows, up to 64 heads (sfa_fwd_mla_g.hip): any top-k the generic kernel takes in one item
+constexpr int kMlaGMaxTopk = 12288;
+bool fwd_mla_g_supported(const Params& p);
+bool fwd_partials_f32(const Params& p);  // the kernel of p writes fp32 split partials (part_of)
+hipError_t launch_fwd_mla_g(const Params& p, hipStream_t s);
+hipError_t launch_combine_f32(const Params& p, hipStream_t s);
 int fwd_d128_idx_cap(const Params& p);
 // d = 128: register-direct gather, 16 heads per wave (sfa_fwd_d128.hip)
 bool fwd_d128_supported(const Params& p);

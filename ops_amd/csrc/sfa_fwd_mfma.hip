@@ -872,14 +872,25 @@ bool mla_supported(const Params& p) {
 
 }  // namespace
 
-// Dispatch over the MFMA forward kernels: the MLA kernel above and the
-// register-direct d = 128 kernel (sfa_fwd_d128.hip).
+// Up to 64 heads on one latent row (one rank of a head-parallel group): the
+// 128-head kernel's 32-head waves would idle and its 256 accumulator
+// registers hold one wave per SIMD, so these have their own kernel.
+bool fwd_mla_g_supported(const Params& p) {
+  return p.Dqk == 576 && p.Dv == 512 && p.G <= 64 && p.topk <= kMlaGMaxTopk && v_is_k_prefix(p) && rows_fit_32bit(p);
+}
+bool fwd_partials_f32(const Params& p) { return fwd_mla_g_supported(p); }
+
+// Dispatch over the MFMA forward kernels: the MLA kernels (above and
+// sfa_fwd_mla_g.hip) and the register-direct d = 128 kernel
+// (sfa_fwd_d128.hip).
 int fwd_mfma_tile_keys(const Params& p) {
   if (p.Dqk == 576 && p.Dv == 512) return CfgMla::NKT;
   return 32;  // d = 128 kernel: 32-key tiles
 }
 
-int fwd_mfma_idx_cap(const Params& p) { return mla_supported(p) ? kIdxCap : fwd_d128_idx_cap(p); }
+int fwd_mfma_idx_cap(const Params& p) {
+  return mla_supported(p) ? kIdxCap : fwd_mla_g_supported(p) ? kMlaGMaxTopk : fwd_d128_idx_cap(p);
+}
 
 // Whether the forward of p runs persistent (its Params then need sched, 8
 // zeroed ints): the MLA kernel without split-k over enough items to keep
@@ -888,14 +899,19 @@ bool fwd_mfma_persistent(const Params& p) {
   return mla_supported(p) && p.num_splits == 1 && (int64_t)p.B * p.Sq * p.Hkv >= 4096;
 }
 
-bool fwd_mfma_supported(const Params& p) { return mla_supported(p) || fwd_d128_supported(p); }
+bool fwd_mfma_supported(const Params& p) {
+  return mla_supported(p) || fwd_mla_g_supported(p) || fwd_d128_supported(p);
+}
 
-// The MLA kernel holds all G heads of an item in one workgroup; the d = 128
+// The MLA kernels hold all G heads of an item in one workgroup; the d = 128
 // kernel one head group of 16.
-int fwd_mfma_head_groups(const Params& p) { return mla_supported(p) ? 1 : fwd_d128_head_groups(p); }
+int fwd_mfma_head_groups(const Params& p) {
+  return mla_supported(p) || fwd_mla_g_supported(p) ? 1 : fwd_d128_head_groups(p);
+}
 
 hipError_t launch_fwd_mfma(const Params& p, hipStream_t s) {
   if (mla_supported(p)) return launch<CfgMla>(p, s);
+  if (fwd_mla_g_supported(p)) return launch_fwd_mla_g(p, s);
   if (fwd_d128_supported(p)) return launch_fwd_d128(p, s);
   return hipErrorNotSupported;
 }

@@ -13,113 +13,25 @@
 // a fixed order by dsink_kernel.
 
 #include "sfa_common.h"
+#include "sfa_generic_row.h"
 
 namespace sfa {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
+constexpr int kThreads = kRowThreads;
+constexpr int kWaves = kRowWaves;
 
-__device__ __forceinline__ float block_reduce_max(float x, float* red) {
-  x = wave_max(x);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[w] = x;
-  __syncthreads();
-  float r = red[0];
-#pragma unroll
-  for (int i = 1; i < kWaves; ++i) r = fmaxf(r, red[i]);
-  return r;
-}
-
-__device__ __forceinline__ float block_reduce_sum(float x, float* red) {
-  x = wave_sum(x);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[w] = x;
-  __syncthreads();
-  float r = 0.f;
-#pragma unroll
-  for (int i = 0; i < kWaves; ++i) r += red[i];
-  return r;
-}
-
-// Shared memory: q row [Dqk] | per-slot score / probability [topk] | reduce [kWaves]
 template <typename T>
 __global__ __launch_bounds__(kThreads) void fwd_generic_kernel(Params p) {
   extern __shared__ float smem[];
-  float* qs = smem;
-  float* sc = smem + p.Dqk;
-  float* red = sc + p.topk;
-
   const int row = blockIdx.x;  // (b, t, h) flattened as ((b*Sq)+t)*Hq+h
   const int h = row % p.Hq;
   const int t = (row / p.Hq) % p.Sq;
   const int b = row / (p.Hq * p.Sq);
-  const int g = h / p.G;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-  const T* qrow = reinterpret_cast<const T*>(p.q) + b * p.q_sb + t * p.q_ss + h * p.q_sh;
-  for (int d = tid; d < p.Dqk; d += kThreads) qs[d] = to_f32(qrow[d]);
-  __syncthreads();
-
-  const int32_t* irow = p.idx + b * p.i_sb + t * p.i_ss + g * p.i_sh;
-  const int bound = bound_of(p, b);
-  // paged KV: k / v are pools and the slot's pool row comes from the block
-  // table (-1 for an invalid slot or an unmapped page)
-  const bool paged = p.block_table != nullptr;
-  const T* kb = reinterpret_cast<const T*>(p.k) + (paged ? 0 : b * p.k_sb) + g * p.k_sh;
-  const T* vb = reinterpret_cast<const T*>(p.v) + (paged ? 0 : b * p.v_sb) + g * p.v_sh;
-  const int pmask = (1 << p.page_shift) - 1;
-  auto key_row = [&](const T* base, int id, int64_t sb, int64_t ss) -> const T* {
-    if (paged) {
-      const int r = paged_row(p, b, id, bound);
-      return r < 0 ? nullptr : base + (int64_t)(r >> p.page_shift) * sb + (int64_t)(r & pmask) * ss;
-    }
-    return (id >= 0 && id < bound) ? base + (int64_t)id * ss : nullptr;
-  };
-
-  for (int j = wave; j < p.topk; j += kWaves) {
-    const T* kr = key_row(kb, irow[j], p.k_sb, p.k_ss);
-    float s = kNegInf;
-    if (kr != nullptr) {
-      float acc = 0.f;
-      for (int d = lane; d < p.Dqk; d += 64) acc += qs[d] * to_f32(kr[d]);
-      s = wave_sum(acc) * p.scale_log2;
-    }
-    if (lane == 0) sc[j] = s;
-  }
-  __syncthreads();
-
-  float m = kNegInf;
-  for (int j = tid; j < p.topk; j += kThreads) m = fmaxf(m, sc[j]);
-  m = block_reduce_max(m, red);
-  const float sink2 = p.sink ? p.sink[h] * kLog2e : kNegInf;
-  const float mm = fmaxf(m, sink2);
-
-  float l = 0.f;
-  for (int j = tid; j < p.topk; j += kThreads) {
-    const float s = sc[j];
-    const float e = (s == kNegInf) ? 0.f : exp2f(s - mm);
-    sc[j] = e;
-    l += e;
-  }
-  l = block_reduce_sum(l, red);  // contains the barrier that publishes sc[]
-  if (p.sink && mm != kNegInf) l += exp2f(sink2 - mm);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-
   T* orow = reinterpret_cast<T*>(p.out) + b * p.o_sb + t * p.o_ss + h * p.o_sh;
-  for (int d = tid; d < p.Dv; d += kThreads) {
-    float acc = 0.f;
-    for (int j = 0; j < p.topk; ++j) {
-      const float e = sc[j];
-      if (e != 0.f) acc += e * to_f32(key_row(vb, irow[j], p.v_sb, p.v_ss)[d]);
-    }
-    orow[d] = from_f32<T>(acc * inv);
-  }
-  if (tid == 0) {
-    p.lse[b * p.l_sb + t * p.l_ss + h * p.l_sh] = (l > 0.f) ? (mm + log2f(l)) * kLn2 : kNegInf;
-  }
+  const float lse2 = generic_fwd_row<T>(p, b, t, h, 0, p.topk, true, smem,
+                                        [&](int d, float x) { orow[d] = from_f32<T>(x); });
+  if (threadIdx.x == 0) p.lse[b * p.l_sb + t * p.l_ss + h * p.l_sh] = lse2 * kLn2;
 }
 
 // δ = Σ_d out·dout per (b, t, h) row (SFA.py:590-610), minus dlse when a

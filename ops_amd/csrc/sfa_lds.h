@@ -108,6 +108,17 @@ __device__ __forceinline__ void gather_tile(const int* ib, u32x4* dst, const __a
 __device__ __forceinline__ int tile_swz(int r) {
   return (((r >> 1) & 1) << 2) ^ ((r >> 2) & 1) ^ (((r >> 3) & 1) << 1);
 }
+struct TileSwz {
+  static __device__ __forceinline__ int at(int r) { return tile_swz(r); }
+};
+// The same for 16x16x32 operands, whose transposing reads (one 32-lane pass)
+// take 8 consecutive rows x an aligned pair of chunks: row bits 1 and 2, the
+// ones that vary among the pass's rows of one bank half, move whole pairs.
+struct TileSwz16 {
+  static __device__ __forceinline__ int at(int r) {
+    return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
+  }
+};
 
 // Row-wise gather for wide rows (PITCH >= 64 slots, so one 64-lane
 // instruction spans at most two rows).  Wave w gathers tile rows
@@ -167,6 +178,11 @@ struct BufRowsUT : BufRows {
   __device__ __forceinline__ void load_lds16(u32x4* dst, base_t off) const { dma_lds16_untracked(rs, dst, off); }
   static constexpr bool kUntrackedDma = true;
 };
+// BufRowsOff with untracked DMA
+struct BufRowsOffUT : BufRowsOff {
+  __device__ __forceinline__ void load_lds16(u32x4* dst, base_t off) const { dma_lds16_untracked(rs, dst, off); }
+  static constexpr bool kUntrackedDma = true;
+};
 // Rows of a paged pool (ids are the scaled pool offsets of staged_pool_off):
 // 64-bit addresses, since a pool may exceed the 4 GiB a buffer offset
 // reaches; padding rows read kZeroRow.
@@ -192,7 +208,7 @@ struct PoolRows {
   static constexpr bool kUntrackedDma = true;  // the caller waits for vmcnt(0) before reading the tile
 };
 
-template <int NKT, int CH, int NWAVES, bool SWZ, class Src = BufRows>
+template <int NKT, int CH, int NWAVES, bool SWZ, class Src = BufRows, class Swz = TileSwz>
 struct RowGather {
   static constexpr int PITCH = SWZ ? CH : CH + 1;
   static constexpr int RPW = NKT / NWAVES;       // rows per wave
@@ -237,10 +253,10 @@ struct RowGather {
     const int r0 = s0 / PITCH, c0 = s0 % PITCH;
     const int bnd = PITCH - c0;
     const uint32_t l16 = 16u * (uint32_t)lane;
-    const uint32_t x0 = SWZ ? l16 ^ (16u * (uint32_t)tile_swz(wave * RPW + r0)) : l16;
+    const uint32_t x0 = SWZ ? l16 ^ (16u * (uint32_t)Swz::at(wave * RPW + r0)) : l16;
     typename Src::base_t a = base[r0] + (16u * (uint32_t)c0 + x0);
     if (bnd < 64 && r0 + 1 < RPW) {
-      const uint32_t x1 = SWZ ? l16 ^ (16u * (uint32_t)tile_swz(wave * RPW + r0 + 1)) : l16;
+      const uint32_t x1 = SWZ ? l16 ^ (16u * (uint32_t)Swz::at(wave * RPW + r0 + 1)) : l16;
       const typename Src::base_t a1 = base[r0 + 1] + (16u * (uint32_t)c0 + x1 - 16u * (uint32_t)PITCH);
       a = lane < bnd ? a : a1;
     }

@@ -1,0 +1,96 @@
+"""MLA rows (576 / 512) with up to 64 query heads, one rank of a head-parallel
+group (``fwd_mla_g_kernel``), against the fp32 oracle.
+
+Tolerance: the output is rounded to bf16 (half an ulp, 2^-8 of the value at
+most once the fp32 sum differs too) and P is kept to 17 bits, so a sum of
+weights 1 over rows of magnitude up to ~5 is off by at most 5 * 2^-17 < 2^-14.
+LSE is an fp32 sum of the score products: 1e-4 absolute."""
+import pytest
+import torch
+
+import ops_amd
+from ops_amd.workloads import page_kv
+from oracle.sfa_oracle import sfa_forward as ref_forward
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _inputs(B, Sq, Skv, Hq, Hkv, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    q = torch.randn((B, Sq, Hq, 576), generator=g, device=DEV).bfloat16()
+    kv = torch.randn((B, Skv, Hkv, 576), generator=g, device=DEV).bfloat16()
+    # any order, padding and out-of-range ids in between, one masked row
+    idx = torch.randint(-Skv // 8, Skv + Skv // 16, (B, Sq, Hkv, K), generator=g, device=DEV, dtype=torch.int32)
+    idx[0, 0, 0] = -1
+    lens = torch.randint(max(1, Skv // 2), Skv + 1, (B,), generator=g, device=DEV, dtype=torch.int32)
+    return q, kv, idx, lens
+
+
+def _check(out, lse, ref):
+    o_ref, l_ref = ref
+    out, lse = out.float().cpu(), lse.cpu()
+    assert bool(((out - o_ref).abs() <= o_ref.abs() * 2.0 ** -8 + 2.0 ** -14).all())
+    fin = torch.isfinite(l_ref)
+    assert torch.equal(torch.isfinite(lse), fin)
+    assert float((lse - l_ref)[fin].abs().max()) <= 1e-4
+
+
+# tile edges (31 / 32 / 33), the 256-slot halves of the staged index ring (255 .. 257, 513, 2049), group edges
+@pytest.mark.parametrize("G,Hkv,K,splits", [
+    (1, 1, 1, 0), (5, 2, 31, 1), (16, 1, 32, 1), (16, 1, 33, 0), (16, 1, 255, 1), (16, 2, 257, 1), (16, 1, 513, 3),
+    (17, 1, 256, 1), (32, 1, 2049, 1), (32, 2, 300, 8), (33, 1, 224, 1), (48, 1, 2049, 5), (64, 1, 700, 1),
+    (64, 1, 96, 2), (16, 1, 2500, 64)])
+def test_heads_and_slots(G, Hkv, K, splits):
+    q, kv, idx, lens = _inputs(3, 3, 900, G * Hkv, Hkv, K, seed=G * 7 + K)
+    sink = torch.linspace(-2.0, 3.0, G * Hkv, device=DEV) if K % 2 else None
+    out = torch.full(q.shape[:3] + (512,), float("nan"), dtype=q.dtype, device=DEV)
+    out, lse = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, kv_lens=lens, attn_sink=sink, num_splits=splits,
+                                   out=out)
+    ref = ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05, kv_lens=lens.cpu(),
+                      sink=None if sink is None else sink.cpu())
+    _check(out, lse, ref)
+
+
+@pytest.mark.parametrize("G,Sq,K,splits", [(16, 3, 600, 0), (32, 1, 2049, 4), (64, 2, 300, 1)])
+def test_paged_is_contiguous(G, Sq, K, splits):
+    q, kv, idx, lens = _inputs(4, Sq, 1024, G, 1, K, seed=G)
+    kp, vp, bt = page_kv(kv, kv[..., :512], 64, seed=3, spare_pages=3)
+    a = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, kv_lens=lens, num_splits=splits)
+    b = ops_amd.sfa_forward_paged(q, kp, vp, bt, idx, 0.05, kv_lens=lens, num_splits=splits)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    bt[1, 3] = -1  # an unmapped page drops its slots
+    drop = idx.clone()
+    drop[1][(drop[1] >= 192) & (drop[1] < 256)] = -1
+    a = ops_amd.sfa_forward(q, kv, kv[..., :512], drop, 0.05, kv_lens=lens, num_splits=splits)
+    b = ops_amd.sfa_forward_paged(q, kp, vp, bt, idx, 0.05, kv_lens=lens, num_splits=splits)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+def test_infinite_rows(splits):
+    """A selected row with an infinite entry: heads whose score is -inf leave
+    it out, heads whose score is +inf have no finite answer, as a scalar
+    evaluation of the sum gives."""
+    q, kv, idx, _ = _inputs(1, 2, 300, 16, 1, 96, seed=1)
+    idx = idx.clamp(0, 298)
+    idx[..., 40] = 299
+    kv[0, 299] = 0
+    kv[0, 299, 0, 7] = float("inf")
+    q[..., 7] = torch.where(torch.arange(16, device=DEV) % 2 == 0, -1.0, 1.0)
+    out, _ = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, num_splits=splits)
+    kv[0, 299] = 0
+    idx[..., 40] = -1
+    o_ref, _ = ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05)
+    err = (out.float().cpu() - o_ref)[:, :, ::2].abs()
+    assert bool((err <= o_ref[:, :, ::2].abs() * 2.0 ** -8 + 2.0 ** -14).all())
+    assert bool(torch.isnan(out[:, :, 1::2]).all())
+
+
+def test_noalloc_splits_to_its_scratch():
+    """The static scratch bounds the split count instead of refusing the call."""
+    q, kv, idx, _ = _inputs(2, 100, 500, 64, 1, 300, seed=5)
+    out = torch.empty(q.shape[:3] + (512,), dtype=q.dtype, device=DEV)
+    lse = torch.empty(q.shape[:3], dtype=torch.float32, device=DEV)
+    ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, num_splits=8, out=out, lse=lse, noalloc=True)
+    _check(out, lse, ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05))

@@ -380,6 +380,13 @@ namespace {
 // top-k 1024: ~4x dense pairs) it is 4.7x faster than the atomics; the
 // per-pair costs put the crossover near 30x dense pairs.  Rules:
 constexpr int64_t kCsrMaxKeysPerTopk = 64;        // Skv <= 64 * top-k (<= ~32x dense pairs causally)
+// d = 64, where the atomics cost half: S = 8192, 16 heads, top-k 512 (16 keys
+// per slot) 0.73 against 1.67 ms, top-k 128 (64) 0.68 against 0.48 ms; and
+// enough (slot, 16 heads) pairs to repay the scheme's fixed 0.4 ms: S = 4096,
+// 16 heads, top-k 256 (2^20 pairs) 0.47 against 0.46 ms, S = 1024, 64 heads,
+// top-k 1024 (2^22) 0.44 against 0.96 ms.
+constexpr int64_t kCsr64MaxKeysPerTopk = 16;
+constexpr int64_t kCsr64MinSlots = int64_t(1) << 21;
 constexpr size_t kCsrMaxWorkspace = size_t(4) << 30;  // CSR arrays + partials <= 4 GiB
 
 // dK/dV scheme actually used: CSR (deterministic) when requested or, for
@@ -393,8 +400,10 @@ bool use_csr(const sfa_bwd_args* a, sfa::Params p) {
   // the deterministic scheme pairs the key-major dK/dV with the dQ kernel,
   // which adds only the repeated-key slots' dK/dV
   if (!(bwd_mfma_ok(a) && sfa::bwd_csr_supported(p) && sfa::bwd_dq_supported(p))) return false;
-  if (a->dkv_mode == SFA_DKV_CSR) return true;
-  if ((int64_t)p.Skv > kCsrMaxKeysPerTopk * p.topk) return false;
+  // (asked for by name it is the d = 128 scheme, as its contract says)
+  if (a->dkv_mode == SFA_DKV_CSR) return p.Dqk == 128;
+  if ((int64_t)p.Skv > (p.Dqk == 64 ? kCsr64MaxKeysPerTopk : kCsrMaxKeysPerTopk) * p.topk) return false;
+  if (p.Dqk == 64 && (int64_t)p.B * p.Sq * p.Hkv * p.topk * ((p.G + 15) / 16) < kCsr64MinSlots) return false;
   sfa::csr_geometry(p);
   return sfa::csr_workspace_bytes(p) <= kCsrMaxWorkspace;
 }

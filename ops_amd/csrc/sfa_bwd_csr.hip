@@ -1,5 +1,5 @@
 // Deterministic dK/dV for the gfx950 sparse flash attention backward
-// (SFA_DKV_CSR), d_qk = d_v = 128 and G = 1, 2, 4, ..., 128 query heads per
+// (SFA_DKV_CSR), d_qk = d_v = 128 (and 64 under SFA_DKV_AUTO) and G = 1, 2, 4, ..., 128 query heads per
 // KV head (a power of two).
 //
 // Reference: `_attn_bwd_dk_dv` / `_inner_dkv` (SFA.py:1005-1145, 719-853)
@@ -43,20 +43,22 @@ namespace {
 constexpr int kKeyBlock = 128;          // keys per key block (4 waves x 32)
 constexpr int kRowBlock = 128;          // query-head rows per query block
 constexpr int kChunk = 128;             // query blocks per workgroup (64 measured slower)
-constexpr int kD = 128;                 // head dim (d_qk = d_v)
-constexpr int kCH = kD / 8;             // 16-byte chunks per row
-constexpr int kTB = kRowBlock * kCH;    // slots per Q or dO block buffer
-static_assert(kTB % 64 == 0 && kCH == 16, "block buffers: 4 rows per DMA instruction");
 
-// Q / dO block rows are stored unpadded (16 slots) with chunk c of row r at
-// slot c ^ blk_swz(r).  Both operand read patterns are then bank-conflict
-// free (64 banks x 4 bytes, 256 bytes per pass):
+// Q / dO block rows (D dims: D / 8 16-byte slots) are stored unpadded with
+// chunk c of row r at slot c ^ blk_swz(r).  Both operand read patterns are
+// then bank-conflict free (64 banks x 4 bytes, 256 bytes per pass):
 //  * b128 reads of one chunk of 16 consecutive rows (S / dP A operands):
-//    blk_swz is a bijection on every 16 consecutive rows;
+//    d = 128: blk_swz is a bijection on every 16 consecutive rows; d = 64, two
+//    rows per 256 bytes: on the 8 of one parity;
 //  * transposing reads of 4 consecutive rows x an aligned group of 4 chunks
-//    (dV / dK A operands): blk_swz(4m + i) = 4 i + (m & 3) sends the group of
-//    each of the 4 rows to a different group.
-__device__ __forceinline__ int blk_swz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
+//    (dV / dK A operands): d = 128: blk_swz(4m + i) = 4 i + (m & 3) sends the
+//    group of each of the 4 rows to a different group; d = 64: the two rows of
+//    one parity differ in bit 1, which selects the group.
+// It depends on r mod 16 only.
+template <int D>
+__device__ __forceinline__ int blk_swz(int r) {
+  return D == 128 ? 4 * (r & 3) + ((r >> 2) & 3) : 4 * ((r >> 1) & 1) + ((r >> 2) & 3);
+}
 
 // A pointer that is the same in every lane, read from the first lane (a
 // buffer descriptor built from it then stays scalar)
@@ -265,7 +267,17 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
 // (r & (G - 1)); swizzled, see blk_swz), each row's lse and δ, and per wave the
 // bitmap word of its 32 keys for each row.  Buffers are separate arrays so
 // reads of one are not made to wait for DMA into the other.
-__global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
+// d = 64: the operands, accumulators and block buffers are half as large (70 KB
+// of LDS), so two workgroups share a CU.  S = 4096, 64 heads on one kv row,
+// top-k 1024: this kernel 0.60 ms and the whole backward 0.80 ms, against 6.14
+// ms with fp32 atomics for every pair.
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Params p_arg) {
+  constexpr int kD = D;                   // head dim (d_qk = d_v)
+  constexpr int kCH = kD / 8;             // 16-byte chunks per row
+  constexpr int kTB = kRowBlock * kCH;    // slots per Q or dO block buffer
+  constexpr int kLR = 64 / kCH;           // rows per DMA instruction
+  static_assert(kD == 128 || kD == 64, "the block layout is written for these");
   typedef Mfma<32> M;
   typedef M::acc_t acc_t;
   __shared__ u32x4 s_q0[kTB];
@@ -377,13 +389,13 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
       uniform_ptr(p.kmap + ((int64_t)b * p.Hkv + g) * p.Sq * p.kmap_w + kb * 4),
       (uint32_t)(4 * ((int64_t)(p.Sq - 1) * p.kmap_w + 4)));
 
-  // Query block qb into one set of buffers: Q / dO rows (32 instructions
-  // each, 4 rows per instruction, wave w issues instructions w, w + 4, ...),
+  // Query block qb into one set of buffers: Q / dO rows (kTB / 64 instructions
+  // each, kLR rows per instruction, wave w issues instructions w, w + 4, ...),
   // lse (wave 0), δ (wave 1), each wave its bitmap words.  Rows of queries
   // >= Sq read out of range (zeros); such rows have an all-zero mask, so they
   // contribute nothing.
-  // A block load in steps: step k < 8 issues Q and dO instruction 4 k + wave,
-  // steps 8 and 9 the lse / δ / mask rows 64 (k - 8) .. +63.  (Spreading the
+  // A block load in steps: step k < kTB / 256 issues Q and dO instruction 4 k +
+  // wave, the last two the lse / δ / mask rows.  (Spreading the
   // steps over the previous block's MFMA stream measured slower than the
   // burst.)
   constexpr int kLoadSteps = kTB / 64 / 4 + kRowBlock / 64;
@@ -391,8 +403,8 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
     const int t0 = qb * nq;
     if (step < kTB / 64 / 4) {
       const int ki = 4 * step + wave;
-      const int r = 4 * ki + (lane >> 4);
-      const int cc = (lane & 15) ^ blk_swz(r);  // slot lane & 15 of row r holds chunk cc
+      const int r = kLR * ki + lane / kCH;
+      const int cc = (lane % kCH) ^ blk_swz<D>(r);  // slot lane % kCH of row r holds chunk cc
       const int t = t0 + (r >> lg), h = r & (G - 1);
       const bool ok = t < p.Sq;
       const uint32_t oq = ok ? (uint32_t)(2 * (t * p.q_ss + h * p.q_sh) + 16 * cc) : kOOB;
@@ -429,7 +441,7 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
   // S / dP A operand of step s: row n, chunk 2 s + g2.
   uint32_t aofs[kD / 16];
 #pragma unroll
-  for (int st = 0; st < kD / 16; ++st) aofs[st] = (uint32_t)(n * kCH + ((2 * st + g2) ^ blk_swz(n))) * 16u;
+  for (int st = 0; st < kD / 16; ++st) aofs[st] = (uint32_t)(n * kCH + ((2 * st + g2) ^ blk_swz<D>(n))) * 16u;
   // dV / dK A operands (transposing reads): lane group gi of each 16 lanes
   // loads row run + (gi >> 2), dims 32 d + mgrp + 4 (gi & 3) .. +3, i.e. chunk
   // 4 d + cl with cl = mgrp / 8 + (gi & 3) / 2, bytes 8 (gi & 1) on; the runs
@@ -444,7 +456,7 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
       const int row = 4 * g2 + rr + 8 * hh;
 #pragma unroll
       for (int d = 0; d < kD / 32; ++d)
-        vofs[hh][d] = (uint32_t)(row * kCH + ((4 * d + cl) ^ blk_swz(row))) * 16u + (uint32_t)(cc4 & 1) * 8u;
+        vofs[hh][d] = (uint32_t)(row * kCH + ((4 * d + cl) ^ blk_swz<D>(row))) * 16u + (uint32_t)(cc4 & 1) * 8u;
     }
   }
   // One query block = 4 tiles of 32 rows.  Tile t: S, dP (16 MFMAs), then P,
@@ -464,7 +476,7 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
     // (inline-asm MFMAs, so the operand reads of step st + PDK stay ahead of
     // the MFMAs of step st); mid(st) runs after step st's two MFMAs.
     auto sdp = [&](int t, acc_t& sa, acc_t& dpa, auto&& mid) {
-      constexpr int NS = kD / 16, PDK = 4;
+      constexpr int NS = kD / 16, PDK = 4;  // mid(i): 8 pieces, 8 / NS per step
       const uint32_t mrow = (uint32_t)(32 * t * kCH) * 16u;
       // start values: S - lse / scale and dP - δ accumulate directly (C-layout
       // element e is row 32 t + 8 (e / 4) + 4 g2 + e % 4)
@@ -504,8 +516,9 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
         }
         prev_a = ad;
         prev_b = vB[st];
-        mid(st);
-        // keep mid(st) between these MFMAs and the next step's (the
+#pragma unroll
+        for (int i = 0; i < 8 / NS; ++i) mid(8 / NS * st + i);
+        // keep the pieces between these MFMAs and the next step's (the
         // scheduler otherwise sinks all of it below the chain)
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -531,7 +544,10 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
         // sa = S - lse / scale, dpa = dP - δ
         const float ex = __builtin_amdgcn_exp2f(sa[e] * p.scale_log2);
         const float pr = __uint_as_float(__float_as_uint(ex) & keep);
-        const float ds = pr * dpa[e];
+        float ds = pr * dpa[e];
+        // (d = 64: the mask again, as an unselected key row may hold anything and
+        // 0 * NaN is NaN; the atomic scheme these shapes had never read it)
+        if constexpr (D == 64) ds = __uint_as_float(__float_as_uint(ds) & keep);
         pp[jj] = (bf16)pr;
         dd[jj] = (bf16)ds;
       }
@@ -547,35 +563,44 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
     // dV^T += dO^T P, dK^T += Q^T dS over tile t's rows in two 16-row steps
     // kk; step kk's B operand (lane group g2) holds rows 32 t + 16 kk + 4 g2 +
     // {0..3} and the same + 8, which the A operand gets from two transposing
-    // reads of those 4-row runs.  Operand i = 8 kk + 2 d + w (w = 0: dO for
+    // reads of those 4-row runs.  Operand i = 2 ND kk + 2 d + w (w = 0: dO for
     // dV, 1: Q for dK); the reads of operand i + PD are issued before MFMA i.
     // mid(i) runs after MFMA i.
+    constexpr int ND = kD / 32, NA = 4 * ND;
     auto dvdk = [&](int t, auto&& mid) {
       const int set = t == kTiles - 1;
       const uint32_t mrow = (uint32_t)(32 * t * kCH) * 16u;
       auto load_a = [&](int i) -> bf16x8 {
-        const int kk = i / 8, d = (i / 2) % 4, w = i % 2;
+        const int kk = i / (2 * ND), d = (i / 2) % ND, w = i % 2;
         const uint32_t rb = mrow + (uint32_t)(16 * kk * kCH) * 16u;
         const u32x4* src = w ? qt : dt;
         const bf16x4 lo = lds_read_tr16(src, vofs[0][d] + rb);
         const bf16x4 hi = lds_read_tr16(src, vofs[1][d] + rb);
         return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       };
-      constexpr int NA = 16, PD = 4;
+      constexpr int PD = 4;
       bf16x8 abuf[PD];
 #pragma unroll
       for (int i = 0; i < PD; ++i) abuf[i] = load_a(i);
 #pragma unroll
       for (int i = 0; i < NA; ++i) {
-        const int kk = i / 8, d = (i / 2) % 4, w = i % 2;
+        const int kk = i / (2 * ND), d = (i / 2) % ND, w = i % 2;
         const bf16x8 a = abuf[i % PD];
         if (i + PD < NA) abuf[i % PD] = load_a(i + PD);
         const bf16x8 bop = w ? db[set][kk] : pb[set][kk];
         acc_t& acc = w ? dkacc[d] : dvacc[d];
-        if (i % 8 < 2)  // first use of pb[kk] / db[kk], written by VALU
-          M::template mma_agpr<true>(a, bop, acc, prev_a, prev_b);
-        else
-          M::template mma_agpr<false>(a, bop, acc, prev_a, prev_b);
+        const bool first = i % (2 * ND) < 2;  // first use of pb[kk] / db[kk], written by VALU
+        if constexpr (D == 64) {  // (accumulators in VGPRs: half as many, and two waves per SIMD share the file)
+          if (first)
+            M::mma_vn(a, bop, acc, prev_a, prev_b);
+          else
+            M::mma_v(a, bop, acc, prev_a, prev_b);
+        } else {
+          if (first)
+            M::template mma_agpr<true>(a, bop, acc, prev_a, prev_b);
+          else
+            M::template mma_agpr<false>(a, bop, acc, prev_a, prev_b);
+        }
         prev_a = a;
         prev_b = bop;
         mid(i);
@@ -597,8 +622,9 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
         const acc_t& dn = dpacc[(mt + 1) & 1];
         pds_load(mt + 1, 0);
         dvdk(mt, [&](int i) {
-          if (i & 1) {
-            pds(mt + 1, i / 2, sn, dn);
+          constexpr int EV = NA / 8;  // MFMAs per piece
+          if (i % EV == EV - 1) {
+            pds(mt + 1, i / EV, sn, dn);
             __builtin_amdgcn_sched_barrier(0);
           }
         });
@@ -625,10 +651,15 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
 
 #pragma unroll
   for (int d = 0; d < kD / 32; ++d) {
-    M::drain(dkacc[d]);
-    M::drain(dvacc[d]);
+    if constexpr (D == 64) {
+      M::drain_v1(dkacc[d]);
+      M::drain_v1(dvacc[d]);
+    } else {
+      M::drain(dkacc[d]);
+      M::drain(dvacc[d]);
+    }
   }
-  // partial [key][dK 128 | dV 128] of this chunk; C layout: lane (key n,
+  // partial [key][dK D | dV D] of this chunk; C layout: lane (key n,
   // group g2), element e = dim 32 d + 8 (e / 4) + 4 g2 + e % 4
   float* part = p.dkv_part + ((bgk * p.max_chunks + c) * kKeyBlock + wave * 32 + n) * (2 * kD);
 #pragma unroll
@@ -650,6 +681,7 @@ __global__ __launch_bounds__(256, 1) void dkv_keymajor_kernel(Params p_arg) {
 }
 
 // ---- 3. chunk partials -> per-key accumulators (chunk order) --------------
+template <int kD>
 __global__ __launch_bounds__(256) void dkv_reduce_kernel(Params p) {
   constexpr int Q4 = 2 * kD / 4;
   const int64_t n4 = (int64_t)p.B * p.Skv * p.Hkv * Q4;
@@ -684,13 +716,13 @@ bool fits31(int64_t bytes) { return bytes > 0 && bytes < (int64_t)kOOB; }
 
 bool bwd_csr_supported(const Params& p) {
   if (!bwd_mfma_supported(p)) return false;  // the query-major dQ kernel
-  if (p.Dqk != kD || p.Dv != kD) return false;
+  if ((p.Dqk != 128 && p.Dqk != 64) || p.Dv != p.Dqk) return false;
   if (p.G < 1 || p.G > kRowBlock || (p.G & (p.G - 1)) != 0) return false;  // a query block holds whole queries
   const int nkb = (p.Skv + kKeyBlock - 1) / kKeyBlock;
   const int64_t w = 4 * (int64_t)nkb;
   if (w > kMaxMapWords) return false;
-  return fits31(2 * ((int64_t)(p.Sq - 1) * p.q_ss + (int64_t)(p.G - 1) * p.q_sh + kD)) &&
-         fits31(2 * ((int64_t)(p.Sq - 1) * p.do_ss + (int64_t)(p.G - 1) * p.do_sh + kD)) &&
+  return fits31(2 * ((int64_t)(p.Sq - 1) * p.q_ss + (int64_t)(p.G - 1) * p.q_sh + p.Dqk)) &&
+         fits31(2 * ((int64_t)(p.Sq - 1) * p.do_ss + (int64_t)(p.G - 1) * p.do_sh + p.Dv)) &&
          fits31(4 * ((int64_t)(p.Sq - 1) * p.l_ss + (int64_t)(p.G - 1) * p.l_sh + 1)) &&
          fits31(4 * ((int64_t)(p.Sq - 1) * p.Hq + p.G)) && fits31(4 * ((int64_t)(p.Sq - 1) * w + 4));
 }
@@ -711,7 +743,7 @@ size_t csr_workspace_bytes(const Params& p) {
   const size_t bg = (size_t)p.B * p.Hkv;
   return al256(bg * p.Sq * p.kmap_w * 4) + al256((size_t)p.B * p.Sq * p.Hkv * p.topk) +
          al256(bg * p.nkb * p.nqb * 4) + al256(bg * p.nkb * (p.max_chunks + 1) * 4) +
-         al256(bg * p.nkb * p.max_chunks * kKeyBlock * 2 * kD * 4) + al256((size_t)2 * p.B * p.Sq * p.Hq * 4) + 256 +
+         al256(bg * p.nkb * p.max_chunks * kKeyBlock * 2 * p.Dqk * 4) + al256((size_t)2 * p.B * p.Sq * p.Hq * 4) + 256 +
          al256(bg * p.nkb * p.max_chunks * 4);
 }
 
@@ -727,7 +759,7 @@ void csr_bind_workspace(Params& p, void* ws) {
   p.bstart = reinterpret_cast<int*>(c);
   c += al256(bg * p.nkb * (p.max_chunks + 1) * 4);
   p.dkv_part = reinterpret_cast<float*>(c);
-  c += al256(bg * p.nkb * p.max_chunks * kKeyBlock * 2 * kD * 4);
+  c += al256(bg * p.nkb * p.max_chunks * kKeyBlock * 2 * p.Dqk * 4);
   p.rowc = reinterpret_cast<float*>(c);
   c += al256((size_t)2 * p.B * p.Sq * p.Hq * 4);
   p.kctr = reinterpret_cast<int*>(c);
@@ -747,16 +779,21 @@ hipError_t launch_csr_index(const Params& p, hipStream_t s) {
 }
 
 hipError_t launch_csr_dkv(const Params& p, hipStream_t s) {
-  // persistent: one workgroup per CU (its LDS use allows one)
+  // persistent: as many workgroups per CU as its LDS use allows
   int dev = 0, cus = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return e;
-  const int64_t units = (int64_t)p.B * p.Hkv * p.nkb * p.max_chunks;
-  const int64_t wgs = units < cus ? units : cus;
-  hipLaunchKernelGGL(dkv_keymajor_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
-  const int64_t n4 = (int64_t)p.B * p.Skv * p.Hkv * (2 * kD / 4);
-  hipLaunchKernelGGL(dkv_reduce_kernel, dim3(grid_stride_blocks(n4)), dim3(256), 0, s, p);
+  const int64_t units = (int64_t)p.B * p.Hkv * p.nkb * p.max_chunks, room = p.Dqk == 64 ? 2 * cus : cus;
+  const dim3 wgs((unsigned)(units < room ? units : room));
+  const dim3 red(grid_stride_blocks((int64_t)p.B * p.Skv * p.Hkv * (2 * p.Dqk / 4)));
+  if (p.Dqk == 64) {
+    hipLaunchKernelGGL(dkv_keymajor_kernel<64>, wgs, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dkv_reduce_kernel<64>, red, dim3(256), 0, s, p);
+  } else {
+    hipLaunchKernelGGL(dkv_keymajor_kernel<128>, wgs, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dkv_reduce_kernel<128>, red, dim3(256), 0, s, p);
+  }
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 // gfx950 dQ (and dsink) kernel of the deterministic backward for d_qk = d_v =
-// 128: register-direct gather, 16 query heads per wave (G > 16 is split into
+// 128 (and 64; the text below describes 128): register-direct gather, 16 query heads per wave (G > 16 is split into
 // head groups of 16, each its own workgroup).
 //
 // Reference: `_attn_bwd_dq_dsink` / `_inner_dq` (SFA.py:856-1002, 613-716).
@@ -31,15 +31,25 @@ namespace {
 
 constexpr int kIdxCapQ = 2048;  // top-k slots a work item may have
 constexpr int kIdxWin = 512;    // slots staged in LDS at a time (a window of the index row)
-constexpr int kQS = 4;          // 128 / 32 contraction steps over the head dim
-constexpr int kDT = 8;          // 128 / 16 dim tiles
-constexpr int kPK = 17;         // K staging row pitch in 16-byte slots (odd: conflict-free reads)
 constexpr int kMaxGroupQ = 256; // query heads per KV head (16 groups of 16)
+
+// Geometry for head dim D = d_qk = d_v (128; 64, as in the forward): steps
+// of 32 dims, dim tiles of 16, 16-byte chunks per row, the staging pitch (odd:
+// conflict-free reads), rows per load instruction.
+template <int D>
+struct DqD {
+  static_assert(D == 64 || D == 128, "head dims of the register-gather kernels");
+  static constexpr int kQS = D / 32, kDT = D / 16, kCH = D / 8, kPK = kCH + 1, kRPI = 64 / kCH;
+};
+
 __device__ __forceinline__ f32x4 mma16x32(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+template <int D>
 __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
+  constexpr int kQS = DqD<D>::kQS, kDT = DqD<D>::kDT, kPK = DqD<D>::kPK, kCH = DqD<D>::kCH;
+  constexpr int kNI = 32 / DqD<D>::kRPI;  // load instructions per 32-row tile
   __shared__ __attribute__((aligned(16))) int s_idx[kIdxWin];
   __shared__ u32x4 s_k[32 * kPK];
   __shared__ u32x4 s_v[32 * kPK];
@@ -47,6 +57,7 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
   const int lane = threadIdx.x;
   const int lt = lane & 15;  // head column / key row within a 16-row M-tile
   const int hq = lane >> 4;  // lane group
+  const int lc = lane % kCH, lr = lane / kCH;  // row-load chunk and row group
 
   // work item and head group; the head groups of an item go to one XCD (its
   // L2 then serves the re-gathered rows)
@@ -99,27 +110,31 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
   const char* kbase = reinterpret_cast<const char*>(p.k) + 2 * (b * p.k_sb + g * p.k_sh);
   const char* vbase = reinterpret_cast<const char*>(p.v) + 2 * (b * p.v_sb + g * p.v_sh);
   const uint32_t krow_bytes = (uint32_t)(2 * p.k_ss), vrow_bytes = (uint32_t)(2 * p.v_ss);
-  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.k_ss + 128)));
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.v_ss + 128)));
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.k_ss + D)));
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.v_ss + D)));
 
 
   // Loads of tile j (K or V rows): instruction i of a lane loads the 16 bytes
-  // at chunk lt of tile row i + 8 hq (4 whole rows per instruction; a lane's 8
-  // rows are consecutive, so their ids are two 16-byte LDS reads).  Invalid
-  // keys read zeros.
-  auto load_rows = [&](int j, bf16x8 (&kr)[8], bf16x8 (&vr)[8]) {
+  // at chunk lc of tile row i + NI lr (whole rows; a lane's NI rows are
+  // consecutive, so their ids are NI / 4 16-byte LDS reads).  Invalid keys
+  // read zeros.
+  auto load_rows = [&](int j, bf16x8 (&kr)[kNI], bf16x8 (&vr)[kNI]) {
     typedef int i32x4 __attribute__((ext_vector_type(4)));
-    const i32x4 id0 = *reinterpret_cast<const i32x4*>(s_idx + 32 * j + 8 * hq);
-    const i32x4 id1 = *reinterpret_cast<const i32x4*>(s_idx + 32 * j + 8 * hq + 4);
-    const int ids[8] = {id0[0], id0[1], id0[2], id0[3], id1[0], id1[1], id1[2], id1[3]};
+    int ids[kNI];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t o = ids[i] >= 0 ? __umul24((uint32_t)ids[i], krow_bytes) + 16u * (uint32_t)lt : kOOB;
+    for (int q = 0; q < kNI / 4; ++q) {
+      const i32x4 x = *reinterpret_cast<const i32x4*>(s_idx + 32 * j + kNI * lr + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ids[4 * q + e] = x[e];
+    }
+#pragma unroll
+    for (int i = 0; i < kNI; ++i) {
+      const uint32_t o = ids[i] >= 0 ? __umul24((uint32_t)ids[i], krow_bytes) + 16u * (uint32_t)lc : kOOB;
       kr[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rk, o, 0, 0));
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t o = ids[i] >= 0 ? __umul24((uint32_t)ids[i], vrow_bytes) + 16u * (uint32_t)lt : kOOB;
+    for (int i = 0; i < kNI; ++i) {
+      const uint32_t o = ids[i] >= 0 ? __umul24((uint32_t)ids[i], vrow_bytes) + 16u * (uint32_t)lc : kOOB;
       vr[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rv, o, 0, 0));
     }
   };
@@ -135,7 +150,7 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
   const uint32_t r1 = r0 + (uint32_t)(16 * kPK) * 16u;
 
   // tile j of the staged window of wt tiles
-  auto step = [&](int j, int wt, bf16x8 (&kr)[8], bf16x8 (&vr)[8]) {
+  auto step = [&](int j, int wt, bf16x8 (&kr)[kNI], bf16x8 (&vr)[kNI]) {
     const int* ib = s_idx + 32 * j;
     const uint32_t vmask = (uint32_t)__ballot(ib[lane & 31] >= 0);
     const bool more = j + 1 < wt;
@@ -148,9 +163,9 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
     // S^T / dP^T A operands (row 16 mt + lt, chunk 4 s + hq) back, then the
     // loads of the next tile into the freed registers
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      *reinterpret_cast<bf16x8*>(&s_k[(i + 8 * hq) * kPK + lt]) = kr[i];
-      *reinterpret_cast<bf16x8*>(&s_v[(i + 8 * hq) * kPK + lt]) = vr[i];
+    for (int i = 0; i < kNI; ++i) {
+      *reinterpret_cast<bf16x8*>(&s_k[(i + kNI * lr) * kPK + lc]) = kr[i];
+      *reinterpret_cast<bf16x8*>(&s_v[(i + kNI * lr) * kPK + lc]) = vr[i];
     }
     if (more) load_rows(j + 1, kr, vr);
 
@@ -210,7 +225,7 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
       s_idx[i] = (id >= 0 && id < bound) ? id : -1;
     }
     __syncthreads();
-    bf16x8 kr[8], vr[8];
+    bf16x8 kr[kNI], vr[kNI];
     load_rows(0, kr, vr);
     for (int j = 0; j < wt; ++j) step(j, wt, kr, vr);
   }
@@ -237,10 +252,11 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
 constexpr int kIdxCapQG = 2048;
 constexpr int kMaxGroupQG = 128;
 
-template <int NW, bool VK>
+template <int D, int NW, bool VK>
 __global__ __launch_bounds__(64 * NW, 2) void bwd_dq_g_kernel(Params p) {
-  constexpr int R = 32 / NW, RI = R / 4, THR = 64 * NW, TS = 32 * kPK;
-  static_assert(R % 4 == 0 && NW * R == 32, "whole 4-row load instructions");
+  constexpr int kQS = DqD<D>::kQS, kDT = DqD<D>::kDT, kPK = DqD<D>::kPK, kCH = DqD<D>::kCH, kRPI = DqD<D>::kRPI;
+  constexpr int R = 32 / NW, RI = R / kRPI, THR = 64 * NW, TS = 32 * kPK;
+  static_assert(R % kRPI == 0 && NW * R == 32, "whole load instructions");
   __shared__ __attribute__((aligned(16))) int s_idx[kIdxCapQG];
   __shared__ u32x4 s_k[2][TS];
   __shared__ u32x4 s_v[2][VK ? 1 : TS];
@@ -288,20 +304,20 @@ __global__ __launch_bounds__(64 * NW, 2) void bwd_dq_g_kernel(Params p) {
   const char* kbase = reinterpret_cast<const char*>(p.k) + 2 * (b * p.k_sb + g * p.k_sh);
   const char* vbase = reinterpret_cast<const char*>(p.v) + 2 * (b * p.v_sb + g * p.v_sh);
   const uint32_t krow_bytes = (uint32_t)(2 * p.k_ss), vrow_bytes = (uint32_t)(2 * p.v_ss);
-  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.k_ss + 128)));
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.v_ss + 128)));
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.k_ss + D)));
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase, (uint32_t)(2 * ((int64_t)(p.Skv - 1) * p.v_ss + D)));
 
-  // rows of tile j this lane loads: instruction i, chunk lt of tile row
-  // wave R + RI hq + i; invalid keys read zeros
-  const int row0 = wave * R + RI * hq;
+  // rows of tile j this lane loads: instruction i, chunk lc of tile row
+  // wave R + RI lr + i; invalid keys read zeros
+  const int lc = lane % kCH, row0 = wave * R + RI * (lane / kCH);
   auto load_rows = [&](int j, bf16x8 (&kr)[RI], bf16x8 (&vr)[RI]) {
 #pragma unroll
     for (int i = 0; i < RI; ++i) {
       const int id = s_idx[32 * j + row0 + i];
-      const uint32_t ko = id >= 0 ? __umul24((uint32_t)id, krow_bytes) + 16u * (uint32_t)lt : kOOB;
+      const uint32_t ko = id >= 0 ? __umul24((uint32_t)id, krow_bytes) + 16u * (uint32_t)lc : kOOB;
       kr[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rk, ko, 0, 0));
       if constexpr (!VK) {
-        const uint32_t vo = id >= 0 ? __umul24((uint32_t)id, vrow_bytes) + 16u * (uint32_t)lt : kOOB;
+        const uint32_t vo = id >= 0 ? __umul24((uint32_t)id, vrow_bytes) + 16u * (uint32_t)lc : kOOB;
         vr[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rv, vo, 0, 0));
       }
     }
@@ -309,8 +325,8 @@ __global__ __launch_bounds__(64 * NW, 2) void bwd_dq_g_kernel(Params p) {
   auto write_rows = [&](int buf, const bf16x8 (&kr)[RI], const bf16x8 (&vr)[RI]) {
 #pragma unroll
     for (int i = 0; i < RI; ++i) {
-      *reinterpret_cast<bf16x8*>(&s_k[buf][(row0 + i) * kPK + lt]) = kr[i];
-      if constexpr (!VK) *reinterpret_cast<bf16x8*>(&s_v[buf][(row0 + i) * kPK + lt]) = vr[i];
+      *reinterpret_cast<bf16x8*>(&s_k[buf][(row0 + i) * kPK + lc]) = kr[i];
+      if constexpr (!VK) *reinterpret_cast<bf16x8*>(&s_v[buf][(row0 + i) * kPK + lc]) = vr[i];
     }
   };
   auto lds_barrier = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
@@ -397,16 +413,21 @@ __global__ __launch_bounds__(64 * NW, 2) void bwd_dq_g_kernel(Params p) {
   }
 }
 
-bool dq_g_supported(const Params& p) { return p.G > 16 && p.G <= kMaxGroupQG && p.topk <= kIdxCapQG; }
+// (d = 64 up to 64 heads: with 8 waves a wave's 4 rows are half an instruction)
+bool dq_g_supported(const Params& p) {
+  return p.G > 16 && p.G <= (p.Dqk == 64 ? 64 : kMaxGroupQG) && p.topk <= kIdxCapQG;
+}
 
 // dK/dV of index slots that repeat an earlier slot's key in their row (p.dup,
 // written by the index inversion; the key-major pass counts each key once
 // per row).  Such slots are absent from ordinary index sets, so this is
 // plain VALU code: one wave per work item scans its flags and, per flagged
-// slot and head, forms S and dP as dot products over the 128 dims (2 per
+// slot and head, forms S and dP as dot products over the D dims (D / 64 per
 // lane), P and dS, and adds P dO and scale dS Q to the key's rows with fp32
 // atomics (SFA.py:719-853 for the math).
+template <int D>
 __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
+  constexpr int E = D / 64;  // dims per lane
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t item = (int64_t)blockIdx.x * 4 + wave;
   if (item >= (int64_t)p.B * p.Sq * p.Hkv) return;  // the whole wave
@@ -416,9 +437,9 @@ __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
   const uint8_t* drow = p.dup + item * p.topk;
   const int32_t* irow = p.idx + b * p.i_sb + t * p.i_ss + g * p.i_sh;
   const int bound = bound_of(p, b);
-  float* const dkb = p.dk_acc + ((int64_t)b * p.Skv * p.Hkv + g) * 128 + 2 * lane;
-  float* const dvb = p.dv_acc + ((int64_t)b * p.Skv * p.Hkv + g) * 128 + 2 * lane;
-  const int64_t acc_row = (int64_t)p.Hkv * 128;
+  float* const dkb = p.dk_acc + ((int64_t)b * p.Skv * p.Hkv + g) * D + E * lane;
+  float* const dvb = p.dv_acc + ((int64_t)b * p.Skv * p.Hkv + g) * D + E * lane;
+  const int64_t acc_row = (int64_t)p.Hkv * D;
   auto wave_sum = [](float x) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -447,9 +468,13 @@ __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
       const int key = __shfl(id, sl, 64);
       const bf16* krow = reinterpret_cast<const bf16*>(p.k) + b * p.k_sb + (int64_t)key * p.k_ss + g * p.k_sh;
       const bf16* vrow = reinterpret_cast<const bf16*>(p.v) + b * p.v_sb + (int64_t)key * p.v_ss + g * p.v_sh;
-      const float k0 = (float)krow[2 * lane], k1 = (float)krow[2 * lane + 1];
-      const float v0 = (float)vrow[2 * lane], v1 = (float)vrow[2 * lane + 1];
-      float dv0 = 0.f, dv1 = 0.f, dk0 = 0.f, dk1 = 0.f;
+      float kk[E], vv[E], dv[E], dk[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        kk[e] = (float)krow[E * lane + e];
+        vv[e] = (float)vrow[E * lane + e];
+        dv[e] = dk[e] = 0.f;
+      }
       for (int hh = 0; hh < p.G; ++hh) {
         const int h = g * p.G + hh;
         const float lse = p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh];
@@ -457,21 +482,29 @@ __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
         const bf16* qrow = reinterpret_cast<const bf16*>(p.q) + b * p.q_sb + t * p.q_ss + (int64_t)h * p.q_sh;
         const bf16* dorow =
             reinterpret_cast<const bf16*>(p.dout) + b * p.do_sb + t * p.do_ss + (int64_t)h * p.do_sh;
-        const float q0 = (float)qrow[2 * lane], q1 = (float)qrow[2 * lane + 1];
-        const float d0 = (float)dorow[2 * lane], d1 = (float)dorow[2 * lane + 1];
-        const float sc = wave_sum(q0 * k0 + q1 * k1);
-        const float dp = wave_sum(d0 * v0 + d1 * v1);
+        float qq[E], dd[E], sq = 0.f, sd = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          qq[e] = (float)qrow[E * lane + e];
+          dd[e] = (float)dorow[E * lane + e];
+          sq += qq[e] * kk[e];
+          sd += dd[e] * vv[e];
+        }
+        const float sc = wave_sum(sq);
+        const float dp = wave_sum(sd);
         const float pr = exp2f(sc * p.scale_log2 - lse * kLog2e);
         const float ds = pr * (dp - p.delta[((int64_t)b * p.Sq + t) * p.Hq + h]);
-        dv0 += pr * d0;
-        dv1 += pr * d1;
-        dk0 += ds * q0;
-        dk1 += ds * q1;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          dv[e] += pr * dd[e];
+          dk[e] += ds * qq[e];
+        }
       }
-      atomicAdd(dvb + (int64_t)key * acc_row, dv0);
-      atomicAdd(dvb + (int64_t)key * acc_row + 1, dv1);
-      atomicAdd(dkb + (int64_t)key * acc_row, dk0 * p.scale);
-      atomicAdd(dkb + (int64_t)key * acc_row + 1, dk1 * p.scale);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        atomicAdd(dvb + (int64_t)key * acc_row + e, dv[e]);
+        atomicAdd(dkb + (int64_t)key * acc_row + e, dk[e] * p.scale);
+      }
     }
   }
 }
@@ -479,39 +512,52 @@ __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
 }  // namespace
 
 bool bwd_dq_supported(const Params& p) {
-  if (p.Dqk != 128 || p.Dv != 128) return false;
+  if ((p.Dqk != 128 && p.Dqk != 64) || p.Dv != p.Dqk) return false;
   if (p.G > kMaxGroupQ || p.G < 1 || p.topk > kIdxCapQ) return false;
-  const int64_t kb = 2 * ((int64_t)(p.Skv - 1) * p.k_ss + 128);
-  const int64_t vb = 2 * ((int64_t)(p.Skv - 1) * p.v_ss + 128);
+  const int64_t kb = 2 * ((int64_t)(p.Skv - 1) * p.k_ss + p.Dqk);
+  const int64_t vb = 2 * ((int64_t)(p.Skv - 1) * p.v_ss + p.Dv);
   return kb < (int64_t)kOOB && vb < (int64_t)kOOB && fits_u24(2 * p.k_ss) && fits_u24(2 * p.v_ss);
 }
 
-hipError_t launch_bwd_dq(const Params& p, hipStream_t s) {
+template <int D>
+static void launch_dq(const Params& p, hipStream_t s) {
   if (dq_g_supported(p)) {
-    const int64_t n = (int64_t)p.B * p.Sq * p.Hkv;
+    const dim3 n((unsigned)((int64_t)p.B * p.Sq * p.Hkv));
     const bool vk = p.v == p.k && p.v_sb == p.k_sb && p.v_ss == p.k_ss && p.v_sh == p.k_sh;
     const int nw = p.G <= 32 ? 2 : p.G <= 64 ? 4 : 8;
-#define SFA_DQG(NW)                                                                                \
-  if (nw == NW) {                                                                                  \
-    if (vk)                                                                                        \
-      hipLaunchKernelGGL((bwd_dq_g_kernel<NW, true>), dim3((unsigned)n), dim3(64 * NW), 0, s, p);  \
-    else                                                                                           \
-      hipLaunchKernelGGL((bwd_dq_g_kernel<NW, false>), dim3((unsigned)n), dim3(64 * NW), 0, s, p); \
-    return hipGetLastError();                                                                      \
+#define SFA_DQG(NW)                                                                     \
+  if (nw == NW) {                                                                       \
+    if (vk)                                                                             \
+      hipLaunchKernelGGL((bwd_dq_g_kernel<D, NW, true>), n, dim3(64 * NW), 0, s, p);    \
+    else                                                                                \
+      hipLaunchKernelGGL((bwd_dq_g_kernel<D, NW, false>), n, dim3(64 * NW), 0, s, p);   \
+    return;                                                                             \
   }
     SFA_DQG(2)
     SFA_DQG(4)
-    SFA_DQG(8)
+    if constexpr (D == 128) {
+      SFA_DQG(8)
+    }
 #undef SFA_DQG
   }
   const int64_t n = (int64_t)p.B * p.Sq * p.Hkv * ((p.G + 15) / 16);
-  hipLaunchKernelGGL(bwd_dq_kernel, dim3((unsigned)n), dim3(64), 0, s, p);
+  hipLaunchKernelGGL(bwd_dq_kernel<D>, dim3((unsigned)n), dim3(64), 0, s, p);
+}
+
+hipError_t launch_bwd_dq(const Params& p, hipStream_t s) {
+  if (p.Dqk == 64)
+    launch_dq<64>(p, s);
+  else
+    launch_dq<128>(p, s);
   return hipGetLastError();
 }
 
 hipError_t launch_bwd_dup(const Params& p, hipStream_t s) {
-  const int64_t n = (int64_t)p.B * p.Sq * p.Hkv;
-  hipLaunchKernelGGL(bwd_dup_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, p);
+  const dim3 grid((unsigned)(((int64_t)p.B * p.Sq * p.Hkv + 3) / 4));
+  if (p.Dqk == 64)
+    hipLaunchKernelGGL(bwd_dup_kernel<64>, grid, dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(bwd_dup_kernel<128>, grid, dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

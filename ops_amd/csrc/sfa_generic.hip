@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kThreads) void delta_kernel(Params p) {
   }
 }
 
-// The same for bf16 rows of DV in {128, 256, 512} elements with 16-byte
+// The same for bf16 rows of DV in {64, 128, 256, 512} elements with 16-byte
 // aligned rows: DV / 8 lanes per row, one 16-byte load of O and of dO each.
 template <int DV>
 __global__ __launch_bounds__(kThreads) void delta_vec_kernel(Params p) {
@@ -408,13 +408,15 @@ hipError_t launch_bwd_delta(const Params& p, int dtype, hipStream_t s) {
   const int64_t rows = (int64_t)p.B * p.Sq * p.Hq;
   const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
   auto al16 = [](const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; };
-  const bool vec = dtype == SFA_DTYPE_BF16 && (p.Dv == 128 || p.Dv == 256 || p.Dv == 512) && al16(p.out) &&
+  const bool vec = dtype == SFA_DTYPE_BF16 && (p.Dv == 64 || p.Dv == 128 || p.Dv == 256 || p.Dv == 512) && al16(p.out) &&
                    al16(p.dout) && p.o_sb % 8 == 0 && p.o_ss % 8 == 0 && p.o_sh % 8 == 0 && p.do_sb % 8 == 0 &&
                    p.do_ss % 8 == 0 && p.do_sh % 8 == 0;
   if (vec) {
     const int rpw = 64 / (p.Dv / 8);
     const dim3 vgrid((unsigned)((rows + (int64_t)kWaves * rpw - 1) / ((int64_t)kWaves * rpw)));
-    if (p.Dv == 128)
+    if (p.Dv == 64)
+      hipLaunchKernelGGL(delta_vec_kernel<64>, vgrid, dim3(kThreads), 0, s, p);
+    else if (p.Dv == 128)
       hipLaunchKernelGGL(delta_vec_kernel<128>, vgrid, dim3(kThreads), 0, s, p);
     else if (p.Dv == 256)
       hipLaunchKernelGGL(delta_vec_kernel<256>, vgrid, dim3(kThreads), 0, s, p);

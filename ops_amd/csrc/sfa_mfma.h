@@ -63,6 +63,7 @@ struct Mfma<32> {
   static __device__ __forceinline__ void drain_v(acc_t& c, const bf16x8& a, const bf16x8& b) {
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(c) : "v"(a), "v"(b));
   }
+  static __device__ __forceinline__ void drain_v1(acc_t& c) { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(c)); }
   // both VGPR accumulators of two interleaved chains (the last MFMA used a, b)
   static __device__ __forceinline__ void drain_v2(acc_t& c0, acc_t& c1, const bf16x8& a, const bf16x8& b) {
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(c0), "+v"(c1) : "v"(a), "v"(b));

@@ -61,8 +61,8 @@ enum {
                           64 * top-k and CSR workspace (bitmap, lists, fp32 partials,
                           which grow as Skv * Sq * G / 16 bytes per batch and kv head)
                           <= 4 GiB; the same scheme at d_qk = d_v = 64 when Skv <=
-                          16 * top-k and the call is large enough to repay its fixed
-                          cost; otherwise ATOMIC                                       */
+                          32 * top-k and the call is large enough to repay its extra
+                          launches; otherwise ATOMIC                                       */
   SFA_DKV_ATOMIC = 1,  /* fp32 atomic adds into a workspace accumulator (SFA.py:853)    */
   SFA_DKV_CSR = 2      /* deterministic: membership bitmap inverted into per-key-block
                           lists of referencing query blocks, key-major recompute, fixed-

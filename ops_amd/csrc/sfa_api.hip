@@ -380,13 +380,13 @@ namespace {
 // top-k 1024: ~4x dense pairs) it is 4.7x faster than the atomics; the
 // per-pair costs put the crossover near 30x dense pairs.  Rules:
 constexpr int64_t kCsrMaxKeysPerTopk = 64;        // Skv <= 64 * top-k (<= ~32x dense pairs causally)
-// d = 64, where the atomics cost half: S = 8192, 16 heads, top-k 512 (16 keys
-// per slot) 0.73 against 1.67 ms, top-k 128 (64) 0.68 against 0.48 ms; and
-// enough (slot, 16 heads) pairs to repay the scheme's fixed 0.4 ms: S = 4096,
-// 16 heads, top-k 256 (2^20 pairs) 0.47 against 0.46 ms, S = 1024, 64 heads,
-// top-k 1024 (2^22) 0.44 against 0.96 ms.
-constexpr int64_t kCsr64MaxKeysPerTopk = 16;
-constexpr int64_t kCsr64MinSlots = int64_t(1) << 21;
+// d = 64, where the atomics cost half (backward, one kv row): S = 8192, 16
+// heads, top-k 256 (32 keys per slot) 0.50 against 0.88 ms, top-k 128 (64) 0.48
+// against 0.48 ms; and enough (slot, 16 heads) pairs to repay the scheme's
+// extra launches: S = 1024, 16 heads, top-k 256 (2^18 pairs) 99 against 131 us,
+// top-k 128 (2^17) 96 against 86 us.
+constexpr int64_t kCsr64MaxKeysPerTopk = 32;
+constexpr int64_t kCsr64MinSlots = int64_t(1) << 18;
 constexpr size_t kCsrMaxWorkspace = size_t(4) << 30;  // CSR arrays + partials <= 4 GiB
 
 // dK/dV scheme actually used: CSR (deterministic) when requested or, for

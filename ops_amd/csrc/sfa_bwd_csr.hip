@@ -15,11 +15,11 @@
 //     have none).  Then, for every key block of 128 keys, the ascending list
 //     of query blocks (128 query-head rows = 128 / G queries) that select at
 //     least one of its keys (`blist`, a per-key-block CSR at block
-//     granularity), with `bstart` marking where each chunk of kChunk
+//     granularity), with `bstart` marking where each chunk of p.chunk
 //     consecutive query blocks (an absolute query range) begins in it.
 //  2. Key-major recompute.  A work unit is a key block (each wave 32 keys, K
 //     and V rows kept in registers) and one chunk: the listed query blocks in
-//     one absolute range of kChunk query blocks.  One persistent workgroup
+//     one absolute range of p.chunk query blocks.  One persistent workgroup
 //     per CU claims units from a counter, longest first and otherwise in
 //     chunk-descending order, so the units that run together are key blocks
 //     of the same query range and read the same query blocks.  Per query block it recomputes, for every (row, key)
@@ -42,7 +42,7 @@ namespace {
 
 constexpr int kKeyBlock = 128;          // keys per key block (4 waves x 32)
 constexpr int kRowBlock = 128;          // query-head rows per query block
-constexpr int kChunk = 128;             // query blocks per workgroup (64 measured slower)
+constexpr int kChunk = 128;             // query blocks per chunk at most (csr_geometry chooses)
 
 // Q / dO block rows (D dims: D / 8 16-byte slots) are stored unpadded with
 // chunk c of row r at slot c ^ blk_swz(r).  Both operand read patterns are
@@ -114,9 +114,6 @@ __global__ __launch_bounds__(256) void csr_blocklist_kernel(Params p) {
   const int64_t bgk = ((int64_t)b * p.Hkv + g) * p.nkb + kb;
   int* list = p.blist + bgk * p.nqb;
   int* start = p.bstart + bgk * (p.max_chunks + 1);
-  constexpr int kCPI = 256 / kChunk;  // chunks per iteration
-  constexpr int kWPC = kChunk / 64;   // waves per chunk
-  static_assert(kCPI * kChunk == 256 && kWPC * 64 == kChunk, "an iteration covers whole chunks of whole waves");
   int total = 0;
   for (int q0 = 0; q0 < p.nqb; q0 += 256) {
     const int qb = q0 + tid;
@@ -135,18 +132,8 @@ __global__ __launch_bounds__(256) void csr_blocklist_kernel(Params p) {
     int pos = total + __popcll(m & ((1ull << lane) - 1ull));
     for (int w = 0; w < wave; ++w) pos += s_cnt[w];
     if (any) list[pos] = qb;
-    // chunk starts: the kChunk query blocks of chunk c0 + i are those of
-    // waves kWPC i .. kWPC (i + 1) - 1 of this iteration
-    const int c0 = q0 / kChunk;
-    if (tid == 0) {
-      int acc = total;
-#pragma unroll
-      for (int i = 0; i < kCPI; ++i) {
-        if (c0 + i <= p.max_chunks) start[c0 + i] = acc;
-#pragma unroll
-        for (int w = 0; w < kWPC; ++w) acc += s_cnt[kWPC * i + w];
-      }
-    }
+    // a chunk starts where its first query block is or would be
+    if (qb < p.nqb && qb % p.chunk == 0) start[qb / p.chunk] = pos;
     total += s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     __syncthreads();
   }
@@ -192,14 +179,14 @@ __global__ __launch_bounds__(256) void csr_scatter_wave_kernel(Params p) {
 // ---- 1c. the key-major kernel's claim order --------------------------------
 // Units u = (chunk, key block, (b, g)) in base order: chunk-descending, then
 // key block, then (b, g).  The non-empty units are listed longest first, in
-// classes of 16 query blocks (a unit of n listed query blocks is in class
-// (kChunk - n) / 16), each class in base order: the full units keep their
+// classes of an eighth of a chunk (a unit of n listed query blocks is in class
+// 8 (chunk - n) / chunk), each class in base order: the full units keep their
 // grouping by query range (the units that run together share their query
 // blocks in L2), and the short ones, claimed last, fill the end of the
 // key-major kernel.  One workgroup: a unit's position is its class's start
 // plus the count of earlier units of its class (ballots, then a prefix over
 // the waves of the tile and the tiles before it).
-constexpr int kClasses = kChunk / 16;
+constexpr int kClasses = 8;
 __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
   __shared__ int s_cnt[16][kClasses];
   __shared__ int s_start[kClasses];
@@ -210,7 +197,7 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
     const int kb = (u % per_chunk) / nbg, bg = (u % per_chunk) % nbg;
     const int* start = p.bstart + ((int64_t)bg * p.nkb + kb) * (p.max_chunks + 1);
     const int n = start[c + 1] - start[c];
-    return n > 0 ? (kChunk - n) / 16 : -1;
+    return n > 0 ? kClasses * (p.chunk - n) / p.chunk : -1;
   };
   // class sizes
   int cnt[kClasses] = {};
@@ -269,8 +256,8 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
 // reads of one are not made to wait for DMA into the other.
 // d = 64: the operands, accumulators and block buffers are half as large (70 KB
 // of LDS), so two workgroups share a CU.  S = 4096, 64 heads on one kv row,
-// top-k 1024: this kernel 0.60 ms and the whole backward 0.80 ms, against 6.14
-// ms with fp32 atomics for every pair.
+// top-k 1024: this kernel 0.42 ms and the whole backward 0.60-0.69 ms, against
+// 6.14 ms with fp32 atomics for every pair.
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Params p_arg) {
   constexpr int kD = D;                   // head dim (d_qk = d_v)
@@ -734,7 +721,26 @@ void csr_geometry(Params& p) {
   while ((1 << p.lg_g) < p.G) ++p.lg_g;  // G is a power of two <= 128
   const int nq = kRowBlock >> p.lg_g;
   p.nqb = (p.Sq + nq - 1) / nq;
-  p.max_chunks = (p.nqb + kChunk - 1) / kChunk;
+  // Query blocks per chunk.  A unit (key block x chunk) is walked by one
+  // workgroup, so the chunk is what a workgroup does in one piece: long ones
+  // amortise the unit's start and write few partials, short ones share the
+  // blocks out evenly (a full unit of 128 takes ~0.4 ms, whatever the call's
+  // size).  By causal (key block, query block) pairs per CU, d = 128, whole
+  // backward in us at chunks of 128 / 64 / 32 / 16 / 8 / 4:
+  //   512 (B 2, S 8192, 32 heads on 2)  3801 3623 3711 3987
+  //   128 (S 4096, 64 on 1)             1300 1234 1156 1192 1352
+  //    32 (B 2, S 2048, 32 on 2)         741  501  444  457  463  542
+  //     8 (S 2048, 16 on 1)              563  331  226  177  191  207
+  //     4 (S 1024, 32 on 2)              544  313  202  149  130  147
+  //   1.5 (S 600, 32 on 8)               187  180  179  170  144  132
+  // (d = 64 has its minima at the same places.)  Below 128 the partials stay
+  // within 1 GiB.
+  const int64_t bg = (int64_t)p.B * p.Hkv, pairs = bg * p.nkb * p.nqb / 2;
+  p.chunk = pairs >= 192 * 256 ? 64 : pairs >= 24 * 256 ? 32 : pairs >= 6 * 256 ? 16 : pairs >= 2 * 256 ? 8 : 4;
+  for (;; p.chunk *= 2) {
+    p.max_chunks = (p.nqb + p.chunk - 1) / p.chunk;
+    if (p.chunk == kChunk || bg * p.nkb * p.max_chunks * kKeyBlock * 2 * p.Dqk * 4 <= (int64_t)1 << 30) break;
+  }
 }
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }

@@ -71,6 +71,7 @@ struct Params {
   int* uorder;        // [B*Hkv*nkb*max_chunks] key-major units in claim order (non-empty ones only)
   int nkb, nqb;       // key blocks (128 keys), query blocks (128 / G queries)
   int lg_g;           // log2(G)
+  int chunk;          // query blocks per chunk
   int max_chunks;     // chunks per key block (query blocks / chunk, rounded up)
 };
 

@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 
 #include "sfa_common.h"
@@ -125,6 +126,24 @@ bool bwd_mfma_ok(const sfa_bwd_args* a) {
   for (int64_t x : s)
     if (x % 8 != 0) return false;
   return true;
+}
+
+// The float32 kernels on the matrix cores: shape, and 16-byte aligned rows.
+bool rows16_f32(std::initializer_list<const void*> ptrs, std::initializer_list<int64_t> strides) {
+  for (const void* x : ptrs)
+    if (!aligned16(x)) return false;
+  for (int64_t x : strides)
+    if (x % 4 != 0) return false;
+  return true;
+}
+bool fwd_f32_ok(const sfa_fwd_args* a, const sfa::Params& p) {
+  return a->dtype == SFA_DTYPE_F32 && sfa::f32_mfma_supported(p) &&
+         rows16_f32({a->q, a->k, a->v, a->out}, {a->q_sb, a->q_ss, a->q_sh, a->k_sb, a->k_ss, a->k_sh, a->v_sb, a->v_ss,
+                                                 a->v_sh, a->o_sb, a->o_ss, a->o_sh});
+}
+bool bwd_f32_ok(const sfa_bwd_args* a, const sfa::Params& p) {
+  return fwd_f32_ok(&a->fwd, p) &&
+         rows16_f32({a->dout, a->dq}, {a->do_sb, a->do_ss, a->do_sh, a->dq_sb, a->dq_ss, a->dq_sh});
 }
 
 struct FwdPlan {
@@ -258,7 +277,7 @@ int run_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, void* workspace, size
   }
   rc = check_generic_fwd(a);
   if (rc != SFA_OK) return rc;
-  e = sfa::launch_fwd_generic(p, a->dtype, s);
+  e = fwd_f32_ok(a, p) ? sfa::launch_fwd_f32(p, s) : sfa::launch_fwd_generic(p, a->dtype, s);
   if (e != hipSuccess) return hip_fail(e, "sfa_fwd (generic)");
   return SFA_OK;
 }
@@ -636,6 +655,15 @@ int sfa_bwd(const sfa_bwd_args* a, void* workspace, size_t workspace_bytes, void
     sfa::csr_bind_workspace(p, (char*)workspace + bwd_base_bytes(f));
   }
 
+  if (bwd_f32_ok(a, p)) {
+    // (v is k whenever MERGE_KV is given at equal widths)
+    sfa::F32Grads gr{(float*)a->dk, merge ? nullptr : (float*)a->dv, a->dk_sb, a->dk_ss, a->dk_sh,
+                     a->dv_sb,      a->dv_ss,                        a->dv_sh};
+    hipError_t e = sfa::launch_bwd_f32(p, gr, s);
+    if (e == hipSuccess) e = sfa::launch_bwd_dsink(p, s);
+    if (e != hipSuccess) return hip_fail(e, "sfa_bwd (f32)");
+    return SFA_OK;
+  }
   hipError_t e = sfa::launch_zero_f32(p.dk_acc, nk, s);
   if (e == hipSuccess) e = sfa::launch_zero_f32(p.dv_acc, nv, s);
   if (e == hipSuccess) e = sfa::launch_bwd_delta(p, f.dtype, s);

@@ -328,6 +328,16 @@ struct IndexerParams {
 namespace sfa {
 hipError_t launch_fwd_generic(const Params& p, int dtype, hipStream_t s);
 hipError_t launch_bwd_generic(const Params& p, int dtype, hipStream_t s);
+// float32, d_qk = d_v = 64 or 128, 16-byte aligned rows (sfa_f32.hip); the
+// backward adds dK / dV into the gradient tensors themselves (dv nullptr: v is
+// k, one gradient), zeroed by its launcher, and writes δ
+struct F32Grads {
+  float *dk, *dv;
+  int64_t dk_sb, dk_ss, dk_sh, dv_sb, dv_ss, dv_sh;
+};
+bool f32_mfma_supported(const Params& p);
+hipError_t launch_fwd_f32(const Params& p, hipStream_t s);
+hipError_t launch_bwd_f32(const Params& p, const F32Grads& gr, hipStream_t s);
 hipError_t launch_zero_f32(float* ptr, size_t n, hipStream_t s);
 hipError_t launch_bwd_delta(const Params& p, int dtype, hipStream_t s);
 hipError_t launch_bwd_dsink(const Params& p, hipStream_t s);  // after launch_bwd_delta

@@ -209,13 +209,15 @@ SFA_API int sfa_fwd(const sfa_fwd_args* a, void* workspace, size_t workspace_byt
  * claim counters and sorted index rows) goes to a static device
  * buffer of SFA_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds
  * until the process ends; a plan that needs more returns SFA_E_WORKSPACE
- * before any device work, except the prefill's sorted index rows: when they
- * do not fit, the rows are walked in their own order (the result then
- * equals sfa_fwd's with SFA_FWD_IDX_SORTED set; bitwise equal to sfa_fwd
- * whenever the sorted rows fit or the rows are already ascending).  `stream` must belong to the current device; the
- * first call on a device resolves the buffer's address (make it before any
- * graph capture).  All calls on one GPU share the buffer: calls that may
- * overlap on one GPU (unordered streams) race. */
+ * before any device work, with two exceptions.  The kernel for up to 64 heads
+ * (and for up to 4 queries of up to 128) on MLA rows is split no further than
+ * its fp32 partials fit.  The prefill's sorted index rows: when they do not
+ * fit, the rows are walked in their own order (the result then equals
+ * sfa_fwd's with SFA_FWD_IDX_SORTED set; bitwise equal to sfa_fwd whenever the
+ * sorted rows fit or the rows are already ascending).  `stream` must belong to
+ * the current device; the first call on a device resolves the buffer's
+ * address (make it before any graph capture).  All calls on one GPU share the
+ * buffer: calls that may overlap on one GPU (unordered streams) race. */
 SFA_API int sfa_fwd_noalloc(const sfa_fwd_args* a, void* stream);
 
 /* Bytes of device workspace sfa_fwd_paged needs for `a` and `pages`. */

@@ -180,6 +180,15 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SI
     } else if (items < kTargetWorkgroups / 2) {
       // decode-like: too few work items to fill the chip -> split the top-k set
       splits = (int)((kTargetWorkgroups / 2 + items - 1) / items);
+      // (the 128-head kernel: one workgroup per CU, so one round of at most 256,
+      // and at most 8 splits: more load Q (147 KB each) and write and merge
+      // partials longer than their tiles take.  Top-k 2048, us per call by
+      // splits: 8 sequences 32 -> 38.4, 8 -> 27.6; 16: 16 -> 34.6, 8 -> 31.1;
+      // 24: 11 -> 54.4, 8 -> 35.8; 64: 8 -> 77.9, 4 -> 65.8)
+      if (sfa::fwd_mla_supported(p) && items <= kTargetWorkgroups / 4) {
+        splits = (int)(kTargetWorkgroups / 2 / items);
+        if (splits > 8) splits = 8;
+      }
       // (the kernel for few heads: at least 4 tiles a split.  Measured at
       // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 33.7 / 23.3 /
       // 20.3 us, 64 splits 38.5 / 35.2 / 24.7 us: shorter splits load more Q

@@ -359,9 +359,11 @@ bool fwd_mfma_persistent(const Params& p);  // needs Params::sched (8 ints of wo
 bool idx_sort_supported(const Params& p);
 hipError_t launch_idx_sort(const Params& p, int32_t* out, hipStream_t s);
 int fwd_mfma_head_groups(const Params& p);  // workgroups per (work item, split): head groups
-// MLA rows, up to 64 heads (sfa_fwd_mla_g.hip): any top-k the generic kernel takes in one item
+// MLA rows, up to 64 heads or a few queries (sfa_fwd_mla_g.hip): any top-k the generic kernel takes in one item
 constexpr int kMlaGMaxTopk = 12288;
+bool fwd_mla_supported(const Params& p);    // the 128-head kernel (sfa_fwd_mfma.hip)
 bool fwd_mla_g_supported(const Params& p);
+int fwd_mla_g_groups(const Params& p);  // workgroups per (item, split)
 bool fwd_partials_f32(const Params& p);  // the kernel of p writes fp32 split partials (part_of)
 hipError_t launch_fwd_mla_g(const Params& p, hipStream_t s);
 hipError_t launch_combine_f32(const Params& p, hipStream_t s);

@@ -866,8 +866,10 @@ bool rows_fit_32bit(const Params& p) {
   return kb < (int64_t)kOOB && vb < (int64_t)kOOB && fits_u24(2 * p.k_ss) && fits_u24(2 * p.v_ss);
 }
 
+}
+namespace {
 bool mla_supported(const Params& p) {
-  return p.Dqk == 576 && p.Dv == 512 && p.G <= 128 && p.G > 64 && v_is_k_prefix(p) && rows_fit_32bit(p);
+  return p.Dqk == 576 && p.Dv == 512 && p.G <= 128 && p.G > 64 && v_is_k_prefix(p) && rows_fit_32bit(p) && !fwd_mla_g_supported(p);
 }
 
 }  // namespace
@@ -876,9 +878,15 @@ bool mla_supported(const Params& p) {
 // 128-head kernel's 32-head waves would idle and its 256 accumulator
 // registers hold one wave per SIMD, so these have their own kernel.
 bool fwd_mla_g_supported(const Params& p) {
-  return p.Dqk == 576 && p.Dv == 512 && p.G <= 64 && p.topk <= kMlaGMaxTopk && v_is_k_prefix(p) && rows_fit_32bit(p);
+  // (128 heads, top-k 2048, us per call at 16 head groups / 8 splits of the
+  // 128-head kernel: 1 sequence 20.6 / 26.6, 4 sequences 25.1 / 28.0, 8
+  // sequences 32.3 / 27.6)
+  const bool few = (int64_t)p.B * p.Sq * p.Hkv <= 4;
+  return p.Dqk == 576 && p.Dv == 512 && (p.G <= 64 || (p.G <= 128 && few)) && p.topk <= kMlaGMaxTopk &&
+         v_is_k_prefix(p) && rows_fit_32bit(p);
 }
 bool fwd_partials_f32(const Params& p) { return fwd_mla_g_supported(p); }
+bool fwd_mla_supported(const Params& p) { return mla_supported(p); }
 
 // Dispatch over the MFMA forward kernels: the MLA kernels (above and
 // sfa_fwd_mla_g.hip) and the register-direct d = 128 kernel
@@ -906,7 +914,7 @@ bool fwd_mfma_supported(const Params& p) {
 // The MLA kernels hold all G heads of an item in one workgroup; the d = 128
 // kernel one head group of 16.
 int fwd_mfma_head_groups(const Params& p) {
-  return mla_supported(p) || fwd_mla_g_supported(p) ? 1 : fwd_d128_head_groups(p);
+  return mla_supported(p) ? 1 : fwd_mla_g_supported(p) ? fwd_mla_g_groups(p) : fwd_d128_head_groups(p);
 }
 
 hipError_t launch_fwd_mfma(const Params& p, hipStream_t s) {

@@ -27,6 +27,9 @@
 // 11 TB/s that whole rows reach there), the matrix cores with 64.  2048
 // queries on 16384 keys, top-k 2048, 16 heads: 0.52 ms, 64.5 ms on the scalar
 // kernel (one workgroup per query and head).
+// Up to 4 queries of 65 to 128 heads (a few sequences' decode step) take it
+// too, 16 heads per workgroup: the 128-head kernel loads all 147 KB of Q in
+// every split before its first product.
 
 #include "sfa_common.h"
 #include "sfa_generic_row.h"
@@ -71,28 +74,29 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
   const int lt = lane & 15, hq = lane >> 4;
   const int kt = wave & 1, role = wave >> 1;       // S^T: key half; dims half (NG = 1) or head groups
 
-  // ---- work item: the splits of one item on one XCD; without splits, runs
-  // of 32 consecutive queries on one XCD (shared keys meet in its L2) --------
+  // ---- work item: its splits and head groups on one XCD (they share its Q or
+  // its rows); a single one: runs of 32 consecutive queries on one XCD (shared
+  // keys meet in its L2) ------------------------------------------------------
   const int64_t nitems = (int64_t)p.B * p.Sq * p.Hkv;
-  int wi = blockIdx.x, split;
-  if (p.num_splits > 1) {
-    const int main_ids = (int)(nitems / 8 * 8) * p.num_splits;
+  const int nhg = (p.G + 16 * NG - 1) / (16 * NG), nsub = p.num_splits * nhg;
+  int wi = blockIdx.x, sub = 0;
+  if (nsub > 1) {
+    const int main_ids = (int)(nitems / 8 * 8) * nsub;
     if (wi < main_ids) {
       const int x = wi % 8, r = wi / 8;
-      split = r % p.num_splits;
-      wi = (r / p.num_splits) * 8 + x;
+      sub = r % nsub;
+      wi = (r / nsub) * 8 + x;
     } else {
       const int r = wi - main_ids;
-      split = r % p.num_splits;
-      wi = (int)(nitems / 8 * 8) + r / p.num_splits;
+      sub = r % nsub;
+      wi = (int)(nitems / 8 * 8) + r / nsub;
     }
-  } else {
-    split = 0;
-    if (wi < nitems / 256 * 256) {
-      const int x = wi % 8, r = wi / 8;
-      wi = ((r / 32) * 8 + x) * 32 + r % 32;
-    }
+  } else if (wi < nitems / 256 * 256) {
+    const int x = wi % 8, r = wi / 8;
+    wi = ((r / 32) * 8 + x) * 32 + r % 32;
   }
+  const int split = sub / nhg, hg0 = (sub % nhg) * 16 * NG;  // split, first head of the group
+  const int gheads = min(p.G - hg0, 16 * NG);
   const int g = wi % p.Hkv;
   wi /= p.Hkv;
   const int t = wi % p.Sq;
@@ -108,7 +112,7 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
   for (int n = 0; n < NGW; ++n) {
     const int hl = 16 * ((NG == 1 ? 0 : role * NGW) + n) + lt;
     const bf16* qrow = reinterpret_cast<const bf16*>(p.q) + b * p.q_sb + t * p.q_ss +
-                       (int64_t)(g * p.G + min(hl, p.G - 1)) * p.q_sh + 8 * hq + (NG == 1 ? role * 288 : 0);
+                       (int64_t)(g * p.G + hg0 + min(hl, gheads - 1)) * p.q_sh + 8 * hq + (NG == 1 ? role * 288 : 0);
 #pragma unroll
     for (int s = 0; s < KS; ++s) qb[n][s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
   }
@@ -295,8 +299,8 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
     l_sum += __shfl_xor(l_sum, 16, 64);
     l_sum = xor32_sum(l_sum);
     const int hl = 16 * n + lt;
-    if (hl >= p.G) continue;
-    const int h = g * p.G + hl;
+    if (hl >= gheads) continue;
+    const int h = g * p.G + hg0 + hl;
     const int64_t row = ((int64_t)b * p.Sq + t) * p.Hq + h;
     const float m_fin = m_used[n];
     float scale_o, lse2;
@@ -343,8 +347,8 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
   if (s_red[0] | s_red[1] | s_red[2] | s_red[3]) {
     static_assert((kDqk + kMlaGMaxTopk + kRowWaves) * 4 <= 2 * TILE * 16, "the scalar loop's scratch fits the tiles");
     float* smem = reinterpret_cast<float*>(s_k);
-    for (int hl = 0; hl < p.G; ++hl) {
-      const int h = g * p.G + hl;
+    for (int hl = 0; hl < gheads; ++hl) {
+      const int h = g * p.G + hg0 + hl;
       const int64_t row = ((int64_t)b * p.Sq + t) * p.Hq + h;
       __syncthreads();
       const float lse2 = generic_fwd_row<bf16>(p, b, t, h, slot0, nslots, !partial, smem, [&](int d, float x) {
@@ -420,9 +424,12 @@ void launch_ng(const Params& p, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
+// Up to 64 heads in one workgroup; more (a handful of sequences) 16 each.
+int fwd_mla_g_groups(const Params& p) { return p.G <= 64 ? 1 : (p.G + 15) / 16; }
+
 hipError_t launch_fwd_mla_g(const Params& p, hipStream_t s) {
-  const dim3 grid((unsigned)((int64_t)p.B * p.Sq * p.Hkv * p.num_splits));
-  if (p.G <= 16)
+  const dim3 grid((unsigned)((int64_t)p.B * p.Sq * p.Hkv * p.num_splits * fwd_mla_g_groups(p)));
+  if (p.G <= 16 || p.G > 64)
     launch_ng<1>(p, grid, s);
   else if (p.G <= 32)
     launch_ng<2>(p, grid, s);

@@ -488,18 +488,20 @@ hipError_t launch_bwd_finish_merged(const Params& p, int dtype, void* dk, int64_
 hipError_t launch_combine(const Params& p, int dtype, hipStream_t s) {
   const int64_t rows = (int64_t)p.B * p.Sq * p.Hq;
   const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
-  if (p.Dv == 512 && (p.num_splits == 2 || p.num_splits == 4 || p.num_splits == 8)) {
-#define SFA_COMBINE512(NS)                                                              \
-  if (p.num_splits == NS) {                                                               \
-    if (dtype == SFA_DTYPE_F32)                                                           \
-      hipLaunchKernelGGL((combine512_kernel<float, NS>), grid, dim3(kThreads), 0, s, p); \
-    else                                                                                  \
-      hipLaunchKernelGGL((combine512_kernel<bf16, NS>), grid, dim3(kThreads), 0, s, p);  \
-    return hipGetLastError();                                                             \
-  }
-    SFA_COMBINE512(2)
-    SFA_COMBINE512(4)
-    SFA_COMBINE512(8)
+  if (p.Dv == 512 && dtype == SFA_DTYPE_BF16 && p.num_splits <= 8) {
+#define SFA_COMBINE512(NS)                                                                             \
+  case NS:                                                                                             \
+    hipLaunchKernelGGL((combine512_kernel<bf16, NS>), grid, dim3(kThreads), 0, s, p);                  \
+    return hipGetLastError();
+    switch (p.num_splits) {
+      SFA_COMBINE512(2)
+      SFA_COMBINE512(3)
+      SFA_COMBINE512(4)
+      SFA_COMBINE512(5)
+      SFA_COMBINE512(6)
+      SFA_COMBINE512(7)
+      SFA_COMBINE512(8)
+    }
 #undef SFA_COMBINE512
   }
   if (p.Dv == 128 && dtype == SFA_DTYPE_BF16 && (p.num_splits == 2 || p.num_splits == 4 || p.num_splits == 8)) {

@@ -94,3 +94,23 @@ def test_noalloc_splits_to_its_scratch():
     lse = torch.empty(q.shape[:3], dtype=torch.float32, device=DEV)
     ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, num_splits=8, out=out, lse=lse, noalloc=True)
     _check(out, lse, ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05))
+
+
+# 65..128 heads: up to 4 queries in groups of 16 heads (the last one partly empty), more on the 128-head kernel with 2
+# to 8 splits of its own choice, each with its merge
+@pytest.mark.parametrize("B,Sq,Hq,Hkv", [(1, 1, 128, 1), (2, 2, 100, 1), (1, 2, 144, 2), (5, 1, 128, 1), (33, 1, 72, 1),
+                                         (37, 1, 128, 1), (43, 1, 128, 1), (52, 1, 80, 1), (86, 1, 128, 1)])
+def test_few_queries_and_default_splits(B, Sq, Hq, Hkv):
+    q, kv, idx, lens = _inputs(B, Sq, 600, Hq, Hkv, 520, seed=B)
+    idx[0, 0, 0] = torch.arange(520, device=DEV)  # (not masked: it may be the only row)
+    sink = torch.linspace(-2.0, 3.0, Hq, device=DEV)
+    out = torch.full(q.shape[:3] + (512,), float("nan"), dtype=q.dtype, device=DEV)
+    out, lse = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, kv_lens=lens, attn_sink=sink, out=out)
+    o_ref, l_ref = ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05, kv_lens=lens.cpu(),
+                               sink=sink.cpu())
+    if B * Sq * Hkv <= 4:
+        _check(out, lse, (o_ref, l_ref))
+    # the 128-head kernel rounds P and its partials to bf16 (2^-9 each, random signs over the slots)
+    assert float((out.float().cpu() - o_ref).norm() / o_ref.norm()) < 2.0 ** -7
+    fin = torch.isfinite(l_ref)
+    assert torch.equal(torch.isfinite(lse.cpu()), fin) and float((lse.cpu() - l_ref)[fin].abs().max()) < 1e-3

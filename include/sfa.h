@@ -87,7 +87,9 @@ enum {
 #define SFA_FWD_IDX_SORTED 1  /* every index row lists its valid keys in ascending order before any
                                  padding (what sfa_indexer_topk writes).  Without it the persistent
                                  MLA prefill (the MLA shape, no split-k, >= 4096 work items,
-                                 top-k <= 2048, Skv <= 65536; contiguous or paged kv) first writes its rows
+                                 top-k <= 2048, Skv <= 65536; contiguous or paged kv) and the MLA prefill
+                                 of up to 32 heads per row (>= 1024 queries, 8192 <= Skv <= 65536,
+                                 512 <= top-k <= 2048) first write their rows
                                  in that order into the workspace (valid keys ascending, then -1; a
                                  row that repeats a key is kept as it is) and walks those: the
                                  queries running together on an XCD then gather the same regions
@@ -189,9 +191,9 @@ SFA_API const char* sfa_last_error(void);
 /* Bytes of device workspace sfa_fwd needs for `a` (0 when none).
  * Replaces the per-launch workspaces of SFA.py:117-120; what remains: the
  * split-k partial results of the decode shape, and for the persistent MLA
- * prefill (>= 4096 work items) 256 bytes of work-claim counters plus, unless
- * SFA_FWD_IDX_SORTED is set, its index rows in ascending order
- * (B * Sq * Hkv * topk int32). */
+ * prefill (>= 4096 work items) 256 bytes of work-claim counters; for MLA
+ * prefills that walk ascending rows, unless SFA_FWD_IDX_SORTED is set, those
+ * rows (B * Sq * Hkv * topk int32). */
 SFA_API size_t sfa_fwd_workspace_size(const sfa_fwd_args* a);
 
 /* Forward: out = softmax(scale * q k[idx]^T) v[idx], lse = log-sum-exp.

@@ -193,7 +193,12 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SI
       // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 33.7 / 23.3 /
       // 20.3 us, 64 splits 38.5 / 35.2 / 24.7 us: shorter splits load more Q
       // and write more partial rows than the idle CUs repay)
-      if (sfa::fwd_partials_f32(p) && splits > (a->topk + 4 * nk - 1) / (4 * nk)) splits = (a->topk + 4 * nk - 1) / (4 * nk);
+      // (two of its workgroups share a CU: a second one per CU pays while a
+      // split keeps 16 tiles; 64 sequences of 64 heads, 2 / 4 splits 82 / 67 us)
+      if (sfa::fwd_partials_f32(p)) {
+        if (a->topk >= 2 * splits * 16 * nk) splits *= 2;
+        if (splits > (a->topk + 4 * nk - 1) / (4 * nk)) splits = (a->topk + 4 * nk - 1) / (4 * nk);
+      }
     }
     // each split must fit the staged index window and hold at least one tile
     const int min_splits = (a->topk + idx_cap - 1) / idx_cap;
@@ -225,15 +230,13 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SI
   if (pl.mfma) {
     p.num_splits = pl.num_splits;
     p.split_len = pl.split_len;
-    if (sfa::fwd_mfma_persistent(p)) {
-      pl.sched_bytes = 256;
-      // the persistent MLA prefill walks ascending rows (L2 sharing between
-      // the queries running together on an XCD); paged KV too (the rows hold
-      // logical keys), so a paged call walks the same slots as a contiguous one
-      if (!(a->flags & SFA_FWD_IDX_SORTED) && sfa::idx_sort_supported(p)) {
-        const size_t bytes = align_up((size_t)a->B * a->Sq * a->Hkv * a->topk * sizeof(int32_t), 256);
-        if (bytes + pl.sched_bytes <= room) pl.sort_bytes = bytes;
-      }
+    if (sfa::fwd_mfma_persistent(p)) pl.sched_bytes = 256;
+    // MLA prefills walk ascending rows (L2 sharing between the queries running
+    // together on an XCD); paged KV too (the rows hold logical keys), so a
+    // paged call walks the same slots as a contiguous one
+    if (!(a->flags & SFA_FWD_IDX_SORTED) && sfa::fwd_mfma_ascending(p)) {
+      const size_t bytes = align_up((size_t)a->B * a->Sq * a->Hkv * a->topk * sizeof(int32_t), 256);
+      if (bytes + pl.sched_bytes <= room) pl.sort_bytes = bytes;
     }
   }
   return pl;

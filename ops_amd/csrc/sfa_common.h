@@ -353,6 +353,7 @@ hipError_t launch_fwd_mfma(const Params& p, hipStream_t s);  // paged when p.blo
 bool fwd_mfma_supported(const Params& p);
 int fwd_mfma_tile_keys(const Params& p);
 int fwd_mfma_idx_cap(const Params& p);  // index slots one work item (split) stages
+bool fwd_mfma_ascending(const Params& p);   // launch_idx_sort before it pays
 bool fwd_mfma_persistent(const Params& p);  // needs Params::sched (8 ints of workspace)
 // index rows in ascending key order, then -1 (sfa_idx_sort.hip): out holds
 // B * Sq * Hkv rows of topk slots, contiguous

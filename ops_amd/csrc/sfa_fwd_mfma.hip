@@ -888,6 +888,17 @@ bool fwd_mla_g_supported(const Params& p) {
 bool fwd_partials_f32(const Params& p) { return fwd_mla_g_supported(p); }
 bool fwd_mla_supported(const Params& p) { return mla_supported(p); }
 
+// Whether p's kernel should walk ascending index rows: the persistent MLA
+// prefill, and the kernel for few heads when many queries run together over
+// more rows than an XCD's 4 MB L2 holds (2048 queries on 16384 keys, 16 / 32
+// heads: 0.53 / 0.67 -> 0.42 / 0.60 ms, the pass itself ~12 us; on 4096 keys
+// 115.1 -> 112.5 us, less than the pass).
+bool fwd_mfma_ascending(const Params& p) {
+  if (p.num_splits != 1 || !idx_sort_supported(p)) return false;
+  return fwd_mfma_persistent(p) || (fwd_mla_g_supported(p) && p.G <= 32 && (int64_t)p.B * p.Sq * p.Hkv >= 1024 &&
+                                    p.Skv >= 8192 && p.topk >= 512);
+}
+
 // Dispatch over the MFMA forward kernels: the MLA kernels (above and
 // sfa_fwd_mla_g.hip) and the register-direct d = 128 kernel
 // (sfa_fwd_d128.hip).

@@ -9,12 +9,13 @@
 // heads a gathered row is used for few products (30 FLOP per byte at 16 heads),
 // so the kernel is built around the gather:
 //  * one workgroup of 4 waves per (batch, query, kv head[, split]) and all its
-//    heads, in NG groups of 16 (the MFMA's N); 32-key tiles of whole 1152-byte
+//    heads (up to 32, NG groups of 16, the MFMA's N; more take a workgroup per
+//    32, on one XCD); 32-key tiles of whole 1152-byte
 //    rows straight into LDS (RowGather), double buffered, 78 KB, so that two
 //    workgroups share a CU and one's products cover the other's waits;
 //  * S^T = K Q^T is divided over the waves by key half and, with 16 heads, by
-//    halves of the 576 dims, with more by head groups: a tile row is read once
-//    or twice from LDS, not once per wave, and a wave keeps 36-144 Q registers;
+//    halves of the 576 dims, with 32 by head group: a tile row is read once or
+//    twice from LDS, not once per wave, and a wave keeps 36 or 72 Q registers;
 //  * the scores go through LDS in the accumulator layout (lane-linear 16-byte
 //    slots, conflict free); every wave forms the whole tile's softmax (the
 //    same values in each) and P^T in the B-operand layout;
@@ -24,9 +25,10 @@
 // ran on held both in fp32, and the result's error against float64 is the same
 // (it is the output's rounding, 1.7e-3).
 // Bound: the gather with 16 heads (9.1 TB/s from the Infinity Cache of the
-// 11 TB/s that whole rows reach there), the matrix cores with 64.  2048
-// queries on 16384 keys, top-k 2048, 16 heads: 0.52 ms, 64.5 ms on the scalar
-// kernel (one workgroup per query and head).
+// 11 TB/s that whole rows reach there; 11.4 TB/s on ascending index rows, part
+// of it from L2), the matrix cores with 64.  2048 queries on 16384 keys, top-k
+// 2048, 16 heads: 0.52 ms, 0.43 ms on ascending rows, 64.5 ms on the scalar
+// kernel (one workgroup per query and head); 64 heads 1.18 ms.
 // Up to 4 queries of 65 to 128 heads (a few sequences' decode step) take it
 // too, 16 heads per workgroup: the 128-head kernel loads all 147 KB of Q in
 // every split before its first product.
@@ -54,46 +56,46 @@ __device__ __forceinline__ void full_barrier() {
 }
 
 template <int NG, bool PAGED>
-__global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params p) {
+__global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
   using M = Mfma<16>;
   typedef M::acc_t acc_t;
   typedef typename std::conditional<PAGED, PoolRows, BufRowsOffUT>::type Src;
   typedef RowGather<kKeys, kCh, 4, true, Src, TileSwz16> RG;
-  constexpr int NGW = NG <= 2 ? 1 : NG / 2;        // head groups of a wave's S^T
+  static_assert(NG == 1 || NG == 2, "S^T is divided over the wave pairs by dims (16 heads) or by head group (32)");
   constexpr int KS = NG == 1 ? 9 : 18;             // contraction steps (32 dims) of a wave's S^T
-  constexpr int NX = NG == 1 ? 2 : NG;             // exchanged score blocks per key half
   constexpr int TILE = kKeys * kCh;                // 16-byte slots
 
   __shared__ u32x4 s_k[2 * TILE];                  // two tiles (the scalar fallback's scratch at the end)
-  __shared__ f32x4 s_x[NX * 2][64];                // [block][key half][lane]
+  __shared__ f32x4 s_x[4][64];                     // [role][key half][lane]
   __shared__ int s_idx[2 * kHalf];                 // ring of staged slots: row offsets, < 0 invalid
   __shared__ int s_red[4];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lt = lane & 15, hq = lane >> 4;
-  const int kt = wave & 1, role = wave >> 1;       // S^T: key half; dims half (NG = 1) or head groups
+  const int kt = wave & 1, role = wave >> 1;       // S^T: key half; dims half (NG = 1) or head group
 
-  // ---- work item: its splits and head groups on one XCD (they share its Q or
-  // its rows); a single one: runs of 32 consecutive queries on one XCD (shared
-  // keys meet in its L2) ------------------------------------------------------
+  // ---- work item: its splits and head groups on one XCD (workgroup id % 8:
+  // they share its Q or its rows), unsplit items in runs of 32 consecutive
+  // queries on one XCD (shared keys meet in its L2) ---------------------------
   const int64_t nitems = (int64_t)p.B * p.Sq * p.Hkv;
   const int nhg = (p.G + 16 * NG - 1) / (16 * NG), nsub = p.num_splits * nhg;
-  int wi = blockIdx.x, sub = 0;
-  if (nsub > 1) {
-    const int main_ids = (int)(nitems / 8 * 8) * nsub;
-    if (wi < main_ids) {
-      const int x = wi % 8, r = wi / 8;
-      sub = r % nsub;
-      wi = (r / nsub) * 8 + x;
-    } else {
-      const int r = wi - main_ids;
-      sub = r % nsub;
-      wi = (int)(nitems / 8 * 8) + r / nsub;
-    }
-  } else if (wi < nitems / 256 * 256) {
-    const int x = wi % 8, r = wi / 8;
+  const int runs = p.num_splits == 1 ? (int)(nitems / 256 * 256) : 0;  // items placed in runs
+  const int eights = (int)((nitems - runs) / 8 * 8);                   // then items placed by eights
+  int wi = blockIdx.x, sub;
+  if (wi < runs * nsub) {
+    const int x = wi % 8, r = wi / 8 / nsub;
+    sub = wi / 8 % nsub;
     wi = ((r / 32) * 8 + x) * 32 + r % 32;
+  } else {
+    const int id = wi - runs * nsub, x = id % 8;
+    if (id < eights * nsub) {
+      sub = id / 8 % nsub;
+      wi = runs + id / 8 / nsub * 8 + x;
+    } else {
+      sub = (id - eights * nsub) % nsub;
+      wi = runs + eights + (id - eights * nsub) / nsub;
+    }
   }
   const int split = sub / nhg, hg0 = (sub % nhg) * 16 * NG;  // split, first head of the group
   const int gheads = min(p.G - hg0, 16 * NG);
@@ -107,14 +109,13 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
   const int bound = bound_of(p, b);
 
   // ---- Q^T B operands: lane holds head 16 ng + lt, dims 32 s + 8 hq ----------
-  bf16x8 qb[NGW][KS];
-#pragma unroll
-  for (int n = 0; n < NGW; ++n) {
-    const int hl = 16 * ((NG == 1 ? 0 : role * NGW) + n) + lt;
+  bf16x8 qb[KS];
+  {
+    const int hl = (NG == 1 ? 0 : 16 * role) + lt;
     const bf16* qrow = reinterpret_cast<const bf16*>(p.q) + b * p.q_sb + t * p.q_ss +
                        (int64_t)(g * p.G + hg0 + min(hl, gheads - 1)) * p.q_sh + 8 * hq + (NG == 1 ? role * 288 : 0);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qb[n][s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
+    for (int s = 0; s < KS; ++s) qb[s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s);
   }
 
   // ---- rows ------------------------------------------------------------------
@@ -220,17 +221,11 @@ __global__ __launch_bounds__(256, NG <= 2 ? 2 : 1) void fwd_mla_g_kernel(Params 
     if (j + 1 < ntiles) gather(j + 1, kn);
 
     // S^T of this wave's keys
-    acc_t sacc[NGW];
+    acc_t sacc{};
 #pragma unroll
-    for (int n = 0; n < NGW; ++n) sacc[n] = acc_t{};
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const bf16x8 a = lds_read_b128(kb, ka[s & 1] + (uint32_t)(s >> 1) * 128u);
-#pragma unroll
-      for (int n = 0; n < NGW; ++n) sacc[n] = M::mma(a, qb[n][s], sacc[n]);
-    }
-#pragma unroll
-    for (int n = 0; n < NGW; ++n) s_x[(role * NGW + n) * 2 + kt][lane] = sacc[n];
+    for (int s = 0; s < KS; ++s)
+      sacc = M::mma(lds_read_b128(kb, ka[s & 1] + (uint32_t)(s >> 1) * 128u), qb[s], sacc);
+    s_x[role * 2 + kt][lane] = sacc;
     lds_barrier();
 
     // softmax of head group n over this lane's 8 keys: key(kt, e) = 16 kt + 4 hq + e
@@ -424,17 +419,18 @@ void launch_ng(const Params& p, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
-// Up to 64 heads in one workgroup; more (a handful of sequences) 16 each.
-int fwd_mla_g_groups(const Params& p) { return p.G <= 64 ? 1 : (p.G + 15) / 16; }
+// Heads per workgroup: 16 for a few queries of many heads, else 32.  Four
+// groups (64 heads in one workgroup, one wave per SIMD) keep each row's gather
+// single but leave the products nothing to overlap with: 2048 queries of 64
+// heads 1.57 against 1.18 ms in two workgroups that meet in their XCD's L2.
+int fwd_mla_g_groups(const Params& p) { return p.G <= 64 ? (p.G + 31) / 32 : (p.G + 15) / 16; }
 
 hipError_t launch_fwd_mla_g(const Params& p, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)p.B * p.Sq * p.Hkv * p.num_splits * fwd_mla_g_groups(p)));
   if (p.G <= 16 || p.G > 64)
     launch_ng<1>(p, grid, s);
-  else if (p.G <= 32)
-    launch_ng<2>(p, grid, s);
   else
-    launch_ng<4>(p, grid, s);
+    launch_ng<2>(p, grid, s);
   return hipGetLastError();
 }
 

@@ -114,3 +114,30 @@ def test_few_queries_and_default_splits(B, Sq, Hq, Hkv):
     assert float((out.float().cpu() - o_ref).norm() / o_ref.norm()) < 2.0 ** -7
     fin = torch.isfinite(l_ref)
     assert torch.equal(torch.isfinite(lse.cpu()), fin) and float((lse.cpu() - l_ref)[fin].abs().max()) < 1e-3
+
+
+@pytest.mark.parametrize("G,Sq", [(16, 1301), (24, 1024), (40, 1301)])
+def test_many_queries(G, Sq):
+    """Unsplit items placed in runs of 32 queries, then by eights, then singly
+    (1301 = 1280 + 16 + 5), up to 32 heads on ascending rows: the sorted rows of
+    the library equal rows sorted by the caller bitwise; sampled rows against
+    the oracle; bitwise the same without allocation where the rows fit."""
+    g = torch.Generator(device=DEV).manual_seed(G)
+    Skv, K = 8200, 520
+    q = torch.randn((1, Sq, G, 576), generator=g, device=DEV).bfloat16()
+    kv = torch.randn((1, Skv, 1, 576), generator=g, device=DEV).bfloat16()
+    idx = torch.stack([torch.randperm(Skv, generator=g, device=DEV)[:K] for _ in range(Sq)]).view(1, Sq, 1, K).int()
+    idx[torch.rand(idx.shape, generator=g, device=DEV) < 0.05] = -1
+    out = torch.full(q.shape[:3] + (512,), float("nan"), dtype=q.dtype, device=DEV)
+    out, lse = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, out=out)
+    rows = torch.cat([torch.arange(0, Sq, 97), torch.arange(Sq - 24, Sq)])
+    ref = ref_forward(q[:, rows.to(DEV)].cpu(), kv.cpu(), kv[..., :512].cpu(), idx[:, rows.to(DEV)].cpu(), 0.05)
+    _check(out[:, rows.to(DEV)], lse[:, rows.to(DEV)], ref)
+    assert bool(torch.isfinite(out).all())
+    if G <= 32:
+        asc = torch.where(idx < 0, Skv, idx).sort(-1).values
+        asc = torch.where(asc == Skv, -1, asc).int()
+        o2, l2 = ops_amd.sfa_forward(q, kv, kv[..., :512], asc, 0.05, idx_sorted=True)
+        assert torch.equal(out, o2) and torch.equal(lse, l2)
+    o3, l3 = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, noalloc=True)
+    assert torch.equal(out, o3) and torch.equal(lse, l3)

@@ -676,18 +676,24 @@ int sfa_bwd(const sfa_bwd_args* a, void* workspace, size_t workspace_bytes, void
     if (e != hipSuccess) return hip_fail(e, "sfa_bwd (f32)");
     return SFA_OK;
   }
+  if (csr) {
+    const sfa::GradOut out{a->dk,    merge ? nullptr : a->dv, a->dk_sb, a->dk_ss, a->dk_sh,
+                           a->dv_sb, a->dv_ss,                a->dv_sh};
+    hipError_t e = sfa::launch_bwd_delta(p, f.dtype, s);
+    if (e == hipSuccess) e = sfa::launch_bwd_dsink(p, s);
+    if (e == hipSuccess) e = sfa::launch_csr_index(p, s);
+    if (e == hipSuccess) e = sfa::launch_bwd_dq(p, s);
+    if (e == hipSuccess) e = sfa::launch_csr_dkv(p, s);
+    if (e == hipSuccess) e = sfa::launch_bwd_dup(p, s);  // into the accumulators the finish adds
+    if (e == hipSuccess) e = sfa::launch_csr_finish(p, out, s);
+    if (e != hipSuccess) return hip_fail(e, "sfa_bwd (key-major)");
+    return SFA_OK;
+  }
   hipError_t e = sfa::launch_zero_f32(p.dk_acc, nk, s);
   if (e == hipSuccess) e = sfa::launch_zero_f32(p.dv_acc, nv, s);
   if (e == hipSuccess) e = sfa::launch_bwd_delta(p, f.dtype, s);
   if (e == hipSuccess) e = sfa::launch_bwd_dsink(p, s);
-  if (e == hipSuccess && csr) e = sfa::launch_csr_index(p, s);  // before dQ: it reads the repeat flags
-  if (e == hipSuccess && csr) {
-    e = sfa::launch_bwd_dq(p, s);
-    if (e == hipSuccess) e = sfa::launch_csr_dkv(p, s);
-    // (after the ordered dK/dV reduction, which adds into the same
-    // accumulators without atomics)
-    if (e == hipSuccess) e = sfa::launch_bwd_dup(p, s);
-  } else if (e == hipSuccess) {
+  if (e == hipSuccess) {
     if (bwd_mfma_ok(a) && sfa::bwd_mfma_supported(p))
       e = sfa::launch_bwd_mfma(p, s);
     else

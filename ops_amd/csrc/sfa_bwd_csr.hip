@@ -31,7 +31,8 @@
 //     order).  Pairs that are not selected get P = 0, so a block costs the
 //     same whatever its density.
 //  3. Reduction.  The chunks of a key block write fp32 partials; a reduction
-//     kernel adds them in chunk order into the per-key accumulators.
+//     kernel adds them in chunk order and writes the bf16 gradients (no cleared
+//     accumulators, no separate conversion: those exist for repeated keys only).
 
 #include "sfa_common.h"
 #include "sfa_lds.h"
@@ -95,6 +96,7 @@ __global__ __launch_bounds__(256) void csr_scatter_kernel(Params p) {
       rep = (atomicOr(&s_map[id >> 5], bit) & bit) ? 1 : 0;
     }
     drow[s] = rep;
+    if (rep) p.kctr[2] = 1;
   }
   __syncthreads();
   for (int w = threadIdx.x; w < p.kmap_w; w += 256) mrow[w] = s_map[w];
@@ -114,6 +116,15 @@ __global__ __launch_bounds__(256) void csr_blocklist_kernel(Params p) {
   const int64_t bgk = ((int64_t)b * p.Hkv + g) * p.nkb + kb;
   int* list = p.blist + bgk * p.nqb;
   int* start = p.bstart + bgk * (p.max_chunks + 1);
+  // the accumulators of this block's keys, which only repeated keys are added to
+  if (p.kctr[2]) {
+    const int keys = min(kKeyBlock, p.Skv - kb * kKeyBlock);
+    for (int i = tid; i < keys * p.Dqk; i += 256) {
+      const int64_t at = (((int64_t)b * p.Skv + kb * kKeyBlock + i / p.Dqk) * p.Hkv + g) * p.Dqk + i % p.Dqk;
+      p.dk_acc[at] = 0.f;
+      p.dv_acc[at] = 0.f;
+    }
+  }
   int total = 0;
   for (int q0 = 0; q0 < p.nqb; q0 += 256) {
     const int qb = q0 + tid;
@@ -169,6 +180,7 @@ __global__ __launch_bounds__(256) void csr_scatter_wave_kernel(Params p) {
       rep = (atomicOr(&map[id >> 5], bit) & bit) ? 1 : 0;
     }
     drow[s] = rep;
+    if (rep) p.kctr[2] = 1;
   }
   __builtin_amdgcn_wave_barrier();
   // kmap_w is a multiple of 4: 16-byte stores
@@ -667,28 +679,61 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
   }  // units
 }
 
-// ---- 3. chunk partials -> per-key accumulators (chunk order) --------------
-template <int kD>
-__global__ __launch_bounds__(256) void dkv_reduce_kernel(Params p) {
-  constexpr int Q4 = 2 * kD / 4;
-  const int64_t n4 = (int64_t)p.B * p.Skv * p.Hkv * Q4;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
+// ---- 3. chunk partials -> bf16 gradients (chunk order) ----------------------
+// Four lanes share 4 dims of a key: lane group u of the wave sums the chunks u,
+// u + 4, ... that wrote a partial (one lane walking all of up to 64 chunks was
+// latency-bound: 44 us for 134 MB), the four sums are added in a fixed tree,
+// then the accumulators if there are repeated keys; with MERGE dK and dV (one
+// gradient of the shared rows).  aligned: 8-byte stores.
+template <int D, bool MERGE>
+__global__ __launch_bounds__(256) void dkv_finish_kernel(Params p, GradOut out, bool aligned) {
+  constexpr int Q4 = (MERGE ? 1 : 2) * D / 4;
+  const int64_t n4 = (int64_t)p.B * p.Skv * p.Hkv * Q4;  // (a multiple of 16)
+  const bool repeats = p.kctr[2] != 0;
+  const int lane = threadIdx.x & 63, sub = lane >> 4;
+  for (int64_t i = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + (lane & 15); i < n4; i += (int64_t)gridDim.x * 64) {
     const int q4 = (int)(i % Q4);
     int64_t r = i / Q4;
     const int g = (int)(r % p.Hkv);
     r /= p.Hkv;
     const int key = (int)(r % p.Skv);
     const int b = (int)(r / p.Skv);
-    const int kb = key / kKeyBlock;
-    const int64_t bgk = ((int64_t)b * p.Hkv + g) * p.nkb + kb;
+    const int64_t bgk = ((int64_t)b * p.Hkv + g) * p.nkb + key / kKeyBlock;
     const int* start = p.bstart + bgk * (p.max_chunks + 1);
-    const float* src = p.dkv_part + (bgk * p.max_chunks * kKeyBlock + (key % kKeyBlock)) * (2 * kD) + 4 * q4;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ch = 0; ch < p.max_chunks; ++ch)  // chunks with entries wrote a partial
-      if (start[ch + 1] > start[ch]) acc += *reinterpret_cast<const f32x4*>(src + (int64_t)ch * kKeyBlock * (2 * kD));
-    const int64_t row = (((int64_t)b * p.Skv + key) * p.Hkv + g) * kD;
-    float* dst = (4 * q4 < kD) ? p.dk_acc + row + 4 * q4 : p.dv_acc + row + 4 * q4 - kD;
-    *reinterpret_cast<f32x4*>(dst) += acc;
+    const float* src = p.dkv_part + (bgk * p.max_chunks * kKeyBlock + (key % kKeyBlock)) * (2 * D) + 4 * q4;
+    f32x4 acc = {}, accv = {};
+#pragma unroll 4
+    for (int ch = sub; ch < p.max_chunks; ch += 4) {
+      if (start[ch + 1] > start[ch]) {
+        acc += *reinterpret_cast<const f32x4*>(src + (int64_t)ch * kKeyBlock * (2 * D));
+        if constexpr (MERGE) accv += *reinterpret_cast<const f32x4*>(src + (int64_t)ch * kKeyBlock * (2 * D) + D);
+      }
+    }
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[e] += __shfl_xor(acc[e], o, 64);
+        if constexpr (MERGE) accv[e] += __shfl_xor(accv[e], o, 64);
+      }
+    if (sub != 0) continue;
+    const bool is_v = !MERGE && 4 * q4 >= D;
+    const int d = is_v ? 4 * q4 - D : 4 * q4;
+    if (repeats) {
+      const int64_t row = (((int64_t)b * p.Skv + key) * p.Hkv + g) * D + d;
+      acc += *reinterpret_cast<const f32x4*>((is_v ? p.dv_acc : p.dk_acc) + row);
+      if constexpr (MERGE) accv += *reinterpret_cast<const f32x4*>(p.dv_acc + row);
+    }
+    if constexpr (MERGE) acc += accv;
+    bf16* dst = is_v ? reinterpret_cast<bf16*>(out.dv) + b * out.dv_sb + key * out.dv_ss + g * out.dv_sh + d
+                     : reinterpret_cast<bf16*>(out.dk) + b * out.dk_sb + key * out.dk_ss + g * out.dk_sh + d;
+    const bf16x4 x = {(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]};
+    if (aligned) {
+      *reinterpret_cast<bf16x4*>(dst) = x;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[e] = x[e];
+    }
   }
 }
 
@@ -792,14 +837,30 @@ hipError_t launch_csr_dkv(const Params& p, hipStream_t s) {
   if (e != hipSuccess) return e;
   const int64_t units = (int64_t)p.B * p.Hkv * p.nkb * p.max_chunks, room = p.Dqk == 64 ? 2 * cus : cus;
   const dim3 wgs((unsigned)(units < room ? units : room));
-  const dim3 red(grid_stride_blocks((int64_t)p.B * p.Skv * p.Hkv * (2 * p.Dqk / 4)));
   if (p.Dqk == 64) {
     hipLaunchKernelGGL(dkv_keymajor_kernel<64>, wgs, dim3(256), 0, s, p);
-    hipLaunchKernelGGL(dkv_reduce_kernel<64>, red, dim3(256), 0, s, p);
   } else {
     hipLaunchKernelGGL(dkv_keymajor_kernel<128>, wgs, dim3(256), 0, s, p);
-    hipLaunchKernelGGL(dkv_reduce_kernel<128>, red, dim3(256), 0, s, p);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_csr_finish(const Params& p, const GradOut& out, hipStream_t s) {
+  const bool merge = out.dv == nullptr;
+  auto al8 = [](const void* x, int64_t a, int64_t b, int64_t c) {
+    return ((uintptr_t)x & 7u) == 0 && a % 4 == 0 && b % 4 == 0 && c % 4 == 0;
+  };
+  const bool aligned = al8(out.dk, out.dk_sb, out.dk_ss, out.dk_sh) && (merge || al8(out.dv, out.dv_sb, out.dv_ss, out.dv_sh));
+  const dim3 grid(grid_stride_blocks(4 * (int64_t)p.B * p.Skv * p.Hkv * ((merge ? 1 : 2) * p.Dqk / 4)));
+#define SFA_FINISH(D, M) hipLaunchKernelGGL((dkv_finish_kernel<D, M>), grid, dim3(256), 0, s, p, out, aligned)
+  if (p.Dqk == 64) {
+    if (merge) SFA_FINISH(64, true);
+    else SFA_FINISH(64, false);
+  } else {
+    if (merge) SFA_FINISH(128, true);
+    else SFA_FINISH(128, false);
+  }
+#undef SFA_FINISH
   return hipGetLastError();
 }
 

@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256) void bwd_dup_kernel(Params p) {
   constexpr int E = D / 64;  // dims per lane
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t item = (int64_t)blockIdx.x * 4 + wave;
-  if (item >= (int64_t)p.B * p.Sq * p.Hkv) return;  // the whole wave
+  if (item >= (int64_t)p.B * p.Sq * p.Hkv || p.kctr[2] == 0) return;  // the whole wave
   const int g = (int)(item % p.Hkv);
   const int t = (int)((item / p.Hkv) % p.Sq);
   const int b = (int)(item / ((int64_t)p.Hkv * p.Sq));

@@ -67,7 +67,8 @@ struct Params {
   int* bstart;        // [B][Hkv][nkb][max_chunks + 1] blist index of each 128-query-block chunk's first entry
   float* dkv_part;    // [B][Hkv][nkb][max_chunks][128][2 D] fp32 partial dK | dV per chunk
   float* rowc;        // [2][B*Sq*Hq] per row: -lse / scale, then -δ (written by the δ pass)
-  int* kctr;          // key-major claims: [0] counter, [1] listed units (both set by unit_order_kernel)
+  int* kctr;          // key-major claims: [0] counter, [1] listed units (both set by unit_order_kernel);
+                      // [2] nonzero if a row repeats a key (cleared by the δ pass, set by the inversion)
   int* uorder;        // [B*Hkv*nkb*max_chunks] key-major units in claim order (non-empty ones only)
   int nkb, nqb;       // key blocks (128 keys), query blocks (128 / G queries)
   int lg_g;           // log2(G)
@@ -402,7 +403,14 @@ void csr_geometry(Params& p);                 // fills kmap_w, nkb, nqb, lg_g, m
 size_t csr_workspace_bytes(const Params& p);  // after csr_geometry
 void csr_bind_workspace(Params& p, void* ws); // carves kmap / dup / blist / bcount / dkv_part / rowc
 hipError_t launch_csr_index(const Params& p, hipStream_t s);  // bitmap, duplicate flags, block lists
-hipError_t launch_csr_dkv(const Params& p, hipStream_t s);    // key-major dK/dV partials + reduction
+hipError_t launch_csr_dkv(const Params& p, hipStream_t s);    // key-major dK/dV partials
+// ... their reduction (plus the accumulators, if a row repeats a key) into the
+// bf16 gradients; dv nullptr: dK + dV into dk
+struct GradOut {
+  void *dk, *dv;
+  int64_t dk_sb, dk_ss, dk_sh, dv_sb, dv_ss, dv_sh;
+};
+hipError_t launch_csr_finish(const Params& p, const GradOut& out, hipStream_t s);
 // top-k index producer: queries [t_begin, t_end) of every sequence
 int indexer_query_block(const IndexerParams& p);
 hipError_t launch_indexer_logits(const IndexerParams& p, int t_begin, int t_end, hipStream_t s);

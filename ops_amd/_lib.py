@@ -124,6 +124,8 @@ def lib_path() -> Path:
 def load() -> ctypes.CDLL:
     """Load libsfa.so once; raises if it is missing or has the wrong ABI."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from .sfa import _opt, _stream
 
 __all__ = ["indexer_topk"]
 
@@ -88,7 +89,5 @@ def indexer_topk(q: torch.Tensor, k: torch.Tensor, weights: torch.Tensor, topk: 
     a.flags = 0
     ws = lib.sfa_indexer_topk_workspace_size(ctypes.byref(a))
     wbuf = torch.empty(ws, dtype=torch.uint8, device=q.device) if ws else None
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    _lib.check(lib.sfa_indexer_topk(ctypes.byref(a), None if wbuf is None else ctypes.c_void_p(wbuf.data_ptr()), ws,
-                                    ctypes.c_void_p(stream)))
+    _lib.check(lib.sfa_indexer_topk(ctypes.byref(a), _opt(wbuf), ws, _stream(q.device)))
     return (idx, logits) if return_logits else idx

@@ -28,6 +28,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import struct
 from typing import Optional, Tuple
 
 import torch
@@ -41,13 +42,33 @@ _DTYPES = {torch.float32: _lib.SFA_DTYPE_F32, torch.bfloat16: _lib.SFA_DTYPE_BF1
 _DKV_MODES = {"auto": _lib.SFA_DKV_AUTO, "atomic": _lib.SFA_DKV_ATOMIC, "csr": _lib.SFA_DKV_CSR}
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
 def _rows(t: torch.Tensor) -> torch.Tensor:
     """The kernels need a unit stride on the feature dimension."""
     return t if t.stride(-1) == 1 else t.contiguous()
+
+
+def _plain(q, k, v, idx, kv_lens, sink, ks=None, vs=None) -> bool:
+    """Whether the call needs neither an error nor a conversion: everything
+    :func:`_validate` asks for, in the types and strides the kernels read.
+    One expression, as an ordinary call evaluates all of it; anything else
+    goes through the checks one by one.  ``ks`` / ``vs``: the logical shapes
+    when ``k`` / ``v`` are page pools."""
+    qs, ids = q.shape, idx.shape
+    ks, vs = ks or k.shape, vs or v.shape
+    if not len(qs) == len(ks) == len(vs) == len(ids) == 4:
+        return False
+    dev, dt = q.device, q.dtype
+    B, Sq, Hq, Dqk = qs
+    _, Skv, Hkv, _ = ks
+    return (dev.type == "cuda" and k.device == dev and v.device == dev and idx.device == dev
+            and dt in _DTYPES and k.dtype == dt and v.dtype == dt and idx.dtype == torch.int32
+            and ks[0] == B and ks[3] == Dqk and vs[0] == B and vs[1] == Skv and vs[2] == Hkv
+            and Hkv > 0 and Hq % Hkv == 0 and ids[0] == B and ids[1] == Sq and ids[2] == Hkv and idx.numel() > 0
+            and q.stride(3) == 1 and k.stride(3) == 1 and v.stride(3) == 1 and idx.stride(3) == 1
+            and (kv_lens is None or (kv_lens.numel() == B and kv_lens.device == dev and kv_lens.dtype == torch.int32
+                                     and kv_lens.is_contiguous()))
+            and (sink is None or (sink.numel() == Hq and sink.device == dev and sink.dtype == torch.float32
+                                  and sink.is_contiguous())))
 
 
 def _validate(q, k, v, idx, kv_lens, sink):
@@ -82,29 +103,37 @@ def _validate(q, k, v, idx, kv_lens, sink):
         raise ValueError("attn_sink must be a [Hq] tensor on q's device")
 
 
-def _fwd_args(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted=False) -> _lib.FwdArgs:
+# sfa_fwd_args / sfa_bwd_args as one format each (native layout, checked against
+# the ctypes mirrors below): packing all fields at once costs a third of
+# setting them one by one.
+_FWD_FMT = "@9if" + 4 * "P3q" + "2P" + 2 * "P3q" + "2i"
+_FWD = struct.Struct(_FWD_FMT)
+_BWD = struct.Struct(_FWD_FMT + 4 * "P3q" + "2P" + "2i")
+assert _FWD.size == ctypes.sizeof(_lib.FwdArgs) and _BWD.size == ctypes.sizeof(_lib.BwdArgs)
+
+
+def _opt(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def _fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted=False, skv=None) -> tuple:
     B, Sq, Hq, Dqk = q.shape
     _, Skv, Hkv, _ = k.shape
-    a = _lib.FwdArgs()
-    a.dtype = _DTYPES[q.dtype]
-    a.B, a.Sq, a.Skv, a.Hq, a.Hkv = B, Sq, Skv, Hq, Hkv
-    a.Dqk, a.Dv, a.topk = Dqk, v.shape[3], idx.shape[3]
-    a.scale = float(scale)
-    a.q, (a.q_sb, a.q_ss, a.q_sh) = q.data_ptr(), q.stride()[:3]
-    a.k, (a.k_sb, a.k_ss, a.k_sh) = k.data_ptr(), k.stride()[:3]
-    a.v, (a.v_sb, a.v_ss, a.v_sh) = v.data_ptr(), v.stride()[:3]
-    a.idx, (a.i_sb, a.i_ss, a.i_sh) = idx.data_ptr(), idx.stride()[:3]
-    a.kv_lens = kv_lens.data_ptr() if kv_lens is not None else None
-    a.sink = sink.data_ptr() if sink is not None else None
-    a.out, (a.o_sb, a.o_ss, a.o_sh) = out.data_ptr(), out.stride()[:3]
-    a.lse, (a.l_sb, a.l_ss, a.l_sh) = lse.data_ptr(), lse.stride()
-    a.num_splits = int(num_splits)
-    a.flags = _lib.SFA_FWD_IDX_SORTED if idx_sorted else 0
-    return a
+    return (_DTYPES[q.dtype], B, Sq, Skv if skv is None else skv, Hq, Hkv, Dqk, v.shape[3], idx.shape[3], float(scale),
+            q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
+            idx.data_ptr(), *idx.stride()[:3], _opt(kv_lens), _opt(sink), out.data_ptr(), *out.stride()[:3],
+            lse.data_ptr(), *lse.stride(), int(num_splits), _lib.SFA_FWD_IDX_SORTED if idx_sorted else 0)
+
+
+def _fwd_args(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted=False, skv=None) -> _lib.FwdArgs:
+    return _lib.FwdArgs.from_buffer_copy(
+        _FWD.pack(*_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted, skv)))
 
 
 def _prep(q, k, v, topk_idxs, kv_lens, sink, validate=True):
     if validate:
+        if _plain(q, k, v, topk_idxs, kv_lens, sink):
+            return q, k, v, topk_idxs, kv_lens, sink
         _validate(q, k, v, topk_idxs, kv_lens, sink)
     q, k, v = _rows(q), _rows(k), _rows(v)
     idx = topk_idxs
@@ -117,6 +146,11 @@ def _prep(q, k, v, topk_idxs, kv_lens, sink, validate=True):
     if sink is not None:
         sink = sink.to(torch.float32).contiguous()
     return q, k, v, idx, kv_lens, sink
+
+
+def _stream(device: torch.device) -> int:
+    """The handle of torch's current stream on ``device``."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def sfa_forward(q, k, v, topk_idxs, sm_scale=None, kv_lens=None, attn_sink=None, num_splits: int = 0,
@@ -140,13 +174,13 @@ def sfa_forward(q, k, v, topk_idxs, sm_scale=None, kv_lens=None, attn_sink=None,
     if lse is None:
         lse = torch.empty((B, Sq, Hq), dtype=torch.float32, device=q.device)
     a = _fwd_args(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted)
-    stream = torch.cuda.current_stream(q.device).cuda_stream
+    ref = ctypes.byref(a)
     if noalloc:
-        _lib.check(lib.sfa_fwd_noalloc(ctypes.byref(a), ctypes.c_void_p(stream)))
+        _lib.check(lib.sfa_fwd_noalloc(ref, _stream(q.device)))
         return out, lse
-    ws = lib.sfa_fwd_workspace_size(ctypes.byref(a))
+    ws = lib.sfa_fwd_workspace_size(ref)
     wbuf = torch.empty(ws, dtype=torch.uint8, device=q.device) if ws else None
-    _lib.check(lib.sfa_fwd(ctypes.byref(a), _ptr(wbuf), ws, ctypes.c_void_p(stream)))
+    _lib.check(lib.sfa_fwd(ref, _opt(wbuf), ws, _stream(q.device)))
     return out, lse
 
 
@@ -180,15 +214,18 @@ def sfa_forward_paged(q, k_cache, v_cache, block_table, topk_idxs, sm_scale=None
     max_pages = block_table.shape[1]
     B = q.shape[0]
     skv = max_pages * page_size
-    # stand-ins of the logical [B, Skv, Hkv, D] caches for the shared
-    # validation (zero-stride; the library gets the pools' strides)
-    kview = k_cache.new_empty(()).expand(B, skv, Hkv, k_cache.shape[3])
-    vview = v_cache.new_empty(()).expand(B, skv, Hkv, v_cache.shape[3])
-    _validate(q, kview, vview, topk_idxs, kv_lens, attn_sink)
-    q, k_cache, v_cache, idx, kv_lens, sink = _prep(q, k_cache.unsqueeze(0), v_cache.unsqueeze(0), topk_idxs,
-                                                    kv_lens, attn_sink, validate=False)
-    k_cache, v_cache = k_cache.squeeze(0), v_cache.squeeze(0)
-    bt = block_table.to(torch.int32)
+    kshape, vshape = (B, skv, Hkv, k_cache.shape[3]), (B, skv, Hkv, v_cache.shape[3])
+    if _plain(q, k_cache, v_cache, topk_idxs, kv_lens, attn_sink, kshape, vshape):
+        idx, sink = topk_idxs, attn_sink
+    else:
+        # stand-ins of the logical [B, Skv, Hkv, D] caches for the shared
+        # validation (zero-stride; the library gets the pools' strides)
+        _validate(q, k_cache.new_empty(()).expand(kshape), v_cache.new_empty(()).expand(vshape), topk_idxs, kv_lens,
+                  attn_sink)
+        q, k_cache, v_cache, idx, kv_lens, sink = _prep(q, k_cache.unsqueeze(0), v_cache.unsqueeze(0), topk_idxs,
+                                                        kv_lens, attn_sink, validate=False)
+        k_cache, v_cache = k_cache.squeeze(0), v_cache.squeeze(0)
+    bt = block_table if block_table.dtype == torch.int32 else block_table.to(torch.int32)
     if bt.stride(-1) != 1:
         bt = bt.contiguous()
     B, Sq, Hq, Dqk = q.shape
@@ -198,18 +235,15 @@ def sfa_forward_paged(q, k_cache, v_cache, block_table, topk_idxs, sm_scale=None
         out = torch.empty((B, Sq, Hq, Dv), dtype=q.dtype, device=q.device)
     if lse is None:
         lse = torch.empty((B, Sq, Hq), dtype=torch.float32, device=q.device)
-    a = _fwd_args(q, kview, vview, idx, out, lse, scale, kv_lens, sink, num_splits)
-    # pools: page, row and head strides
-    a.k, (a.k_sb, a.k_ss, a.k_sh) = k_cache.data_ptr(), k_cache.stride()[:3]
-    a.v, (a.v_sb, a.v_ss, a.v_sh) = v_cache.data_ptr(), v_cache.stride()[:3]
+    # (pools: page, row and head strides)
+    a = _fwd_args(q, k_cache, v_cache, idx, out, lse, scale, kv_lens, sink, num_splits, skv=skv)
     pg = _lib.KvPages()
     pg.block_table = bt.data_ptr()
     pg.bt_sb = bt.stride(0)
     pg.max_pages, pg.page_size, pg.num_pages, pg.flags = max_pages, page_size, num_pages, 0
     ws = lib.sfa_fwd_paged_workspace_size(ctypes.byref(a), ctypes.byref(pg))
     wbuf = torch.empty(ws, dtype=torch.uint8, device=q.device) if ws else None
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    _lib.check(lib.sfa_fwd_paged(ctypes.byref(a), ctypes.byref(pg), _ptr(wbuf), ws, ctypes.c_void_p(stream)))
+    _lib.check(lib.sfa_fwd_paged(ctypes.byref(a), ctypes.byref(pg), _opt(wbuf), ws, _stream(q.device)))
     return out, lse
 
 
@@ -249,10 +283,13 @@ def sfa_backward(q, k, v, topk_idxs, out, lse, dout, sm_scale=None, kv_lens=None
     if merge_kv:
         if not _is_prefix_view(k, v):
             raise ValueError("merge_kv needs v to be the first Dv dims of k's rows (a prefix view of k)")
-        _validate(q, k, v, topk_idxs, kv_lens, attn_sink)
-        k = _rows(k)
-        v = k[..., : v.shape[3]]
-        q, k, v, idx, kv_lens, sink = _prep(q, k, v, topk_idxs, kv_lens, attn_sink, validate=False)
+        if _plain(q, k, v, topk_idxs, kv_lens, attn_sink):
+            idx, sink = topk_idxs, attn_sink
+        else:
+            _validate(q, k, v, topk_idxs, kv_lens, attn_sink)
+            k = _rows(k)
+            v = k[..., : v.shape[3]]
+            q, k, v, idx, kv_lens, sink = _prep(q, k, v, topk_idxs, kv_lens, attn_sink, validate=False)
     else:
         q, k, v, idx, kv_lens, sink = _prep(q, k, v, topk_idxs, kv_lens, attn_sink)
     B, Sq, Hq, Dqk = q.shape
@@ -260,7 +297,7 @@ def sfa_backward(q, k, v, topk_idxs, out, lse, dout, sm_scale=None, kv_lens=None
     Dv = v.shape[3]
     if tuple(dout.shape) != (B, Sq, Hq, Dv) or tuple(out.shape) != (B, Sq, Hq, Dv):
         raise ValueError("out / grad_out must be [B, Sq, Hq, Dv]")
-    dout = _rows(dout.to(q.dtype))
+    dout = _rows(dout if dout.dtype == q.dtype else dout.to(q.dtype))
     out = _rows(out)
     lse = lse.contiguous()
     scale = (1.0 / math.sqrt(Dqk)) if sm_scale is None else float(sm_scale)
@@ -280,21 +317,15 @@ def sfa_backward(q, k, v, topk_idxs, out, lse, dout, sm_scale=None, kv_lens=None
     dsink = torch.empty((Hq,), dtype=torch.float32, device=q.device) if sink is not None else None
     if dlse is not None:
         dlse = dlse.to(torch.float32).contiguous()
-    a = _lib.BwdArgs()
-    a.fwd = _fwd_args(q, k, v, idx, out, lse, scale, kv_lens, sink, 0)
-    a.dout, (a.do_sb, a.do_ss, a.do_sh) = dout.data_ptr(), dout.stride()[:3]
-    a.dq, (a.dq_sb, a.dq_ss, a.dq_sh) = dq.data_ptr(), dq.stride()[:3]
-    a.dk, (a.dk_sb, a.dk_ss, a.dk_sh) = dk.data_ptr(), dk.stride()[:3]
-    if dv is not None:
-        a.dv, (a.dv_sb, a.dv_ss, a.dv_sh) = dv.data_ptr(), dv.stride()[:3]
-    a.dlse = dlse.data_ptr() if dlse is not None else None
-    a.dsink = dsink.data_ptr() if dsink is not None else None
-    a.dkv_mode = _DKV_MODES[mode]
-    a.flags = _lib.SFA_BWD_MERGE_KV if merge_kv else 0
-    ws = lib.sfa_bwd_workspace_size(ctypes.byref(a))
+    a = _lib.BwdArgs.from_buffer_copy(_BWD.pack(
+        *_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, 0), dout.data_ptr(), *dout.stride()[:3],
+        dq.data_ptr(), *dq.stride()[:3], dk.data_ptr(), *dk.stride()[:3], _opt(dv),
+        *((0, 0, 0) if dv is None else dv.stride()[:3]), _opt(dlse), _opt(dsink), _DKV_MODES[mode],
+        _lib.SFA_BWD_MERGE_KV if merge_kv else 0))
+    ref = ctypes.byref(a)
+    ws = lib.sfa_bwd_workspace_size(ref)
     wbuf = torch.empty(ws, dtype=torch.uint8, device=q.device) if ws else None
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    _lib.check(lib.sfa_bwd(ctypes.byref(a), _ptr(wbuf), ws, ctypes.c_void_p(stream)))
+    _lib.check(lib.sfa_bwd(ref, _opt(wbuf), ws, _stream(q.device)))
     return dq, dk, dv, dsink
 
 

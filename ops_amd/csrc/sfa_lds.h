@@ -18,6 +18,12 @@ __device__ __forceinline__ float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// the same over lanes l and l ^ 16 (v_permlane16_swap)
+__device__ __forceinline__ float xor16_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // max of three floats as one v_max3_f32 (fmaxf on values the compiler cannot
 // prove canonical, such as MFMA results from inline asm, adds a quieting
 // v_max x, x per operand; NaN-free inputs here)

@@ -87,9 +87,9 @@ enum {
 #define SFA_FWD_IDX_SORTED 1  /* every index row lists its valid keys in ascending order before any
                                  padding (what sfa_indexer_topk writes).  Without it the persistent
                                  MLA prefill (the MLA shape, no split-k, >= 4096 work items,
-                                 top-k <= 2048, Skv <= 65536; contiguous or paged kv) and the MLA prefill
-                                 of up to 32 heads per row (>= 1024 queries, 8192 <= Skv <= 65536,
-                                 512 <= top-k <= 2048) first write their rows
+                                 top-k <= 2048, Skv <= 65536; contiguous or paged kv) and MLA prefills of
+                                 >= 1024 queries with 8192 <= Skv <= 65536 and top-k <= 2048 (65..128
+                                 heads: >= 1024; up to 32 heads: >= 512) first write their rows
                                  in that order into the workspace (valid keys ascending, then -1; a
                                  row that repeats a key is kept as it is) and walks those: the
                                  queries running together on an XCD then gather the same regions

@@ -69,6 +69,9 @@ __global__ __launch_bounds__(64, 2) void bwd_dq_kernel(Params p) {
     const int x = wi % 8, r = wi / 8;
     hs = r % nhs;
     wi = (r / nhs) * 8 + x;
+  } else if (nhs == 1) {
+    hs = 0;
+    wi = xcd_item(p, wi);
   } else {
     hs = wi % nhs;
     wi /= nhs;

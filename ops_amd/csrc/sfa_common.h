@@ -46,7 +46,6 @@ struct Params {
   int num_splits;
   int split_len;      // slots per split (multiple of the key tile)
   __bf16* part_o;     // [num_splits][B*Sq*Hq][Dv] bf16, normalised by the split's own sum
-  float* part_of;     // the same in fp32 (fwd_partials_f32), instead of part_o
   float* part_lse;    // [num_splits][B*Sq*Hq], base-2 log-sum-exp of the split (-inf if empty)
   int* sched;         // persistent forward: 8 claim counters (one per XCD), zeroed before the launch
   // backward
@@ -72,8 +71,9 @@ struct Params {
   int* uorder;        // [B*Hkv*nkb*max_chunks] key-major units in claim order (non-empty ones only)
   int nkb, nqb;       // key blocks (128 keys), query blocks (128 / G queries)
   int lg_g;           // log2(G)
-  int chunk;          // query blocks per chunk
   int max_chunks;     // chunks per key block (query blocks / chunk, rounded up)
+  int chunk;          // query blocks per chunk
+  float* part_of;     // split partials in fp32 (fwd_partials_f32), instead of part_o
 };
 
 typedef __bf16 bf16;
@@ -95,6 +95,22 @@ __device__ __forceinline__ int bound_of(const Params& p, int b) {
   if (p.kv_lens == nullptr) return p.Skv;
   int n = p.kv_lens[b];
   return n < p.Skv ? n : p.Skv;
+}
+
+// Workgroup id -> work item ((b Sq + t) Hkv + g) of a launch of one workgroup
+// per item.  Workgroups go to the 8 XCDs in turn (id % 8), each with a 4 MB L2:
+//  * with 2, 4 or 8 kv heads an XCD works on one of them, so that its L2
+//    holds that head's rows only;
+//  * the XCDs of a head get runs of 32 consecutive queries in turn, whose
+//    common keys (a recency window) meet in L2; queries that do not fill a
+//    round of runs follow one by one.
+__device__ __forceinline__ int xcd_item(const Params& p, int id) {
+  const int lh = p.Hkv == 8 ? 3 : p.Hkv == 4 ? 2 : p.Hkv == 2 ? 1 : 0;  // log2 of the heads told apart
+  const int nq = (int)((unsigned)p.B * p.Sq * p.Hkv >> lh);
+  const int runs = nq & -(256 >> lh);  // queries in runs (a round: 32 on each of a head's 8 >> lh XCDs)
+  if (id >= runs << lh) return id;
+  const int x = id & 7, r = id >> 3;
+  return (((((r >> 5) << (3 - lh)) + (x >> lh)) << 5) + (r & 31) << lh) + (x & ((1 << lh) - 1));
 }
 
 // Pool row (page * page_size + offset) of logical key id of sequence b in

@@ -87,10 +87,9 @@ __global__ __launch_bounds__(64, 3) void fwd_d128_kernel(Params p) {
     const int x = wi % 8, r = wi / 8;
     sub = r % nsub;
     wi = (r / nsub) * 8 + x;
-  } else if (nsub == 1 && nitems % 256 == 0) {
-    const int x = wi % 8, r = wi / 8;
+  } else if (nsub == 1) {
     sub = 0;
-    wi = ((r / 32) * 8 + x) * 32 + r % 32;
+    wi = xcd_item(p, wi);
   } else {
     sub = wi % nsub;
     wi /= nsub;

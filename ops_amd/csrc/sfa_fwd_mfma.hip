@@ -892,11 +892,13 @@ bool fwd_mla_supported(const Params& p) { return mla_supported(p); }
 // prefill, and the kernel for few heads when many queries run together over
 // more rows than an XCD's 4 MB L2 holds (2048 queries on 16384 keys, 16 / 32
 // heads: 0.53 / 0.67 -> 0.42 / 0.60 ms, the pass itself ~12 us; on 4096 keys
-// 115.1 -> 112.5 us, less than the pass).
+// 115.1 -> 112.5 us, less than the pass), as for 128 heads below the
+// persistent kernel's 4096 queries (2048 on 16384 keys: 1082 -> 1045 us).
 bool fwd_mfma_ascending(const Params& p) {
   if (p.num_splits != 1 || !idx_sort_supported(p)) return false;
-  return fwd_mfma_persistent(p) || (fwd_mla_g_supported(p) && p.G <= 32 && (int64_t)p.B * p.Sq * p.Hkv >= 1024 &&
-                                    p.Skv >= 8192 && p.topk >= 512);
+  if (fwd_mfma_persistent(p)) return true;
+  const bool many = (int64_t)p.B * p.Sq * p.Hkv >= 1024 && p.Skv >= 8192;
+  return many && ((fwd_mla_g_supported(p) && p.G <= 32 && p.topk >= 512) || (mla_supported(p) && p.topk >= 1024));
 }
 
 // Dispatch over the MFMA forward kernels: the MLA kernels (above and

@@ -59,7 +59,7 @@ enum {
   SFA_DKV_AUTO = 0,    /* CSR where supported (bf16, d_qk = d_v = 128, G a power of two
                           <= 128, top-k <= 2048, Skv <= 262144) and cheaper: Skv <=
                           64 * top-k and CSR workspace (bitmap, lists, fp32 partials,
-                          which grow as Skv * Sq * G / 16 bytes per batch and kv head)
+                          Skv * Sq * G / 16 bytes per batch and kv head and more, up to 1 GiB, in small calls)
                           <= 4 GiB; the same scheme at d_qk = d_v = 64 when Skv <=
                           32 * top-k and the call is large enough to repay its extra
                           launches; otherwise ATOMIC                                       */

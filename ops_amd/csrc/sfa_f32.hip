@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256) void bwd_f32_kernel(Params p, F32Grads gr) {
   const float* const o0 = reinterpret_cast<const float*>(p.out) + it.b * p.o_sb + it.t * p.o_ss + (int64_t)it.h0 * p.o_sh;
 
   // B operands over dims (head n, dims 16 j + 4 hq + e) and over heads (head
-  // 4 s + hq, dim 16 j + n; absent heads zero), δ and the softmax's constants
+  // 4 s + hq, dim 16 j + n; rows without a gradient zero), δ and the softmax's constants
   const bool live = n < it.nh;
   const int64_t hn = live ? n : it.nh - 1;
   f32x4 q[J], dob[J];
@@ -299,24 +299,27 @@ __global__ __launch_bounds__(256) void bwd_f32_kernel(Params p, F32Grads gr) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) delta += dob[j][e] * ov[e];
   }
-  float qh[4][J], doh[4][J];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const int64_t hh = 4 * s + hq;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      qh[s][j] = hh < it.nh ? q0[hh * p.q_sh + 16 * j + n] : 0.f;
-      doh[s][j] = hh < it.nh ? d0[hh * p.do_sh + 16 * j + n] : 0.f;
-    }
-  }
   delta += __shfl_xor(delta, 16, 64);
   delta += __shfl_xor(delta, 32, 64);
   const int64_t lofs = it.b * p.l_sb + it.t * p.l_ss + (it.h0 + hn) * p.l_sh;
   if (p.dlse) delta -= p.dlse[lofs];
   if (wave == 0 && hq == 0 && live) p.delta[((int64_t)it.b * p.Sq + it.t) * p.Hq + it.h0 + n] = delta;
   const float lse = p.lse[lofs];
-  // (a row with no valid slot and no sink, or an absent head: P = 0)
-  const float lse2 = live && lse != kNegInf ? lse * kLog2e : __builtin_huge_valf();
+  // (a row with no valid slot and no sink, or an absent head, has no gradient:
+  // its operands are zeros and its dQ is written as zeros, since 0 x inf is not 0)
+  const bool row_live = live && lse != kNegInf;
+  const float lse2 = lse * kLog2e;
+  float qh[4][J], doh[4][J];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int64_t hh = 4 * s + hq;
+    const bool on = __shfl((int)row_live, 4 * s + hq, 64);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      qh[s][j] = on ? q0[hh * p.q_sh + 16 * j + n] : 0.f;
+      doh[s][j] = on ? d0[hh * p.do_sh + 16 * j + n] : 0.f;
+    }
+  }
 
   f32x4 dq[V][4];
 #pragma unroll
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(256) void bwd_f32_kernel(Params p, F32Grads gr) {
       f32x4 pr, ds;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool ok = s_row[16 * kt + 4 * hq + e] >= 0;
+        const bool ok = row_live && s_row[16 * kt + 4 * hq + e] >= 0;
         pr[e] = ok ? exp2f(s[e] * p.scale_log2 - lse2) : 0.f;
         ds[e] = ok ? p.scale * (pr[e] * (dp[e] - delta)) : 0.f;
       }
@@ -423,6 +426,7 @@ __global__ __launch_bounds__(256) void bwd_f32_kernel(Params p, F32Grads gr) {
           f32x4{dq[v][0][e2], dq[v][1][e2], dq[v][2][e2], dq[v][3][e2]};
   __syncthreads();
   const int hs = tid >> 4, c = tid & 15;
+  const bool on = __shfl((int)row_live, hs, 64);
   if (hs >= it.nh) return;
   float* dqrow = reinterpret_cast<float*>(p.dq) + it.b * p.dq_sb + it.t * p.dq_ss + (int64_t)(it.h0 + hs) * p.dq_sh;
 #pragma unroll
@@ -431,7 +435,7 @@ __global__ __launch_bounds__(256) void bwd_f32_kernel(Params p, F32Grads gr) {
     f32x4 x = *reinterpret_cast<const f32x4*>(s_mem + hs * D + d);
 #pragma unroll
     for (int w = 1; w < 4; ++w) x += *reinterpret_cast<const f32x4*>(s_mem + (w * kHeads + hs) * D + d);
-    *reinterpret_cast<f32x4*>(dqrow + d) = x;
+    *reinterpret_cast<f32x4*>(dqrow + d) = on ? x : f32x4{};
   }
 }
 

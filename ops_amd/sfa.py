@@ -112,6 +112,13 @@ _BWD = struct.Struct(_FWD_FMT + 4 * "P3q" + "2P" + "2i")
 assert _FWD.size == ctypes.sizeof(_lib.FwdArgs) and _BWD.size == ctypes.sizeof(_lib.BwdArgs)
 
 
+def _packed(fmt: struct.Struct, *fields) -> bytes:
+    try:
+        return fmt.pack(*fields)
+    except struct.error as e:  # e.g. an out / lse of another rank
+        raise ValueError(f"the call's arguments do not fit the kernels' interface: {e}") from None
+
+
 def _opt(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -127,7 +134,7 @@ def _fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_so
 
 def _fwd_args(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted=False, skv=None) -> _lib.FwdArgs:
     return _lib.FwdArgs.from_buffer_copy(
-        _FWD.pack(*_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted, skv)))
+        _packed(_FWD, *_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, num_splits, idx_sorted, skv)))
 
 
 def _prep(q, k, v, topk_idxs, kv_lens, sink, validate=True):
@@ -317,8 +324,8 @@ def sfa_backward(q, k, v, topk_idxs, out, lse, dout, sm_scale=None, kv_lens=None
     dsink = torch.empty((Hq,), dtype=torch.float32, device=q.device) if sink is not None else None
     if dlse is not None:
         dlse = dlse.to(torch.float32).contiguous()
-    a = _lib.BwdArgs.from_buffer_copy(_BWD.pack(
-        *_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, 0), dout.data_ptr(), *dout.stride()[:3],
+    a = _lib.BwdArgs.from_buffer_copy(_packed(
+        _BWD, *_fwd_fields(q, k, v, idx, out, lse, scale, kv_lens, sink, 0), dout.data_ptr(), *dout.stride()[:3],
         dq.data_ptr(), *dq.stride()[:3], dk.data_ptr(), *dk.stride()[:3], _opt(dv),
         *((0, 0, 0) if dv is None else dv.stride()[:3]), _opt(dlse), _opt(dsink), _DKV_MODES[mode],
         _lib.SFA_BWD_MERGE_KV if merge_kv else 0))

@@ -94,3 +94,20 @@ def test_infinite_rows_and_pages():
     q[..., 3] = -1.0
     got, want = ops_amd.sfa_forward(q, k, v, idx)[0], ops_amd.sfa_forward(q, k, v, drop)[0]
     assert _rel(got, want.cpu()) < TOL
+
+
+def test_rows_without_a_finite_score_have_no_gradient():
+    """A query whose only selected key scores -inf has lse = -inf: its dq is 0
+    and it adds nothing to dk / dv, whatever the key's rows hold."""
+    q, k, v, do, idx, _ = _inputs(1, 4, 64, 8, 1, 64, 20, seed=6)
+    idx = idx.clamp(0, 62)
+    q[0, 2, :, 3] = -1.0
+    k[0, 63] = 0
+    k[0, 63, 0, 3] = float("inf")
+    v[0, 63] = float("inf")
+    idx[0, 2] = -1
+    idx[0, 2, 0, 5] = 63
+    out, lse = ops_amd.sfa_forward(q, k, v, idx)
+    assert bool((lse[0, 2] == -float("inf")).all()) and bool((out[0, 2] == 0).all())
+    dq, dk, dv, _ = ops_amd.sfa_backward(q, k, v, idx, out, lse, do)
+    assert bool((dq[0, 2] == 0).all()) and all(bool(torch.isfinite(x).all()) for x in (dq, dk, dv))

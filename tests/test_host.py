@@ -72,3 +72,16 @@ def test_kv_merge_only_for_views_autograd_tracks():
     assert not m(kv, kv[..., :8], True, False)                 # v's gradient not wanted
     assert not m(kv, kv[..., 4:12], True, True)                # not a prefix of the rows
     assert not m(kv, kv[:, :3, :, :8], True, True)             # fewer rows than k
+
+
+def test_arguments_that_do_not_fit_are_value_errors():
+    """An lse of another rank is a ValueError, as every argument the interface
+    refuses; a scale past float32 becomes infinite, which the library refuses."""
+    q = torch.zeros(1, 2, 4, 64)
+    k = torch.zeros(1, 8, 1, 64)
+    idx = torch.zeros(1, 2, 1, 4, dtype=torch.int32)
+    out, lse = torch.zeros(1, 2, 4, 64), torch.zeros(1, 2, 4)
+    assert sfa._fwd_args(q, k, k, idx, out, lse, 1.0, None, None, 0).Skv == 8
+    with pytest.raises(ValueError):
+        sfa._fwd_args(q, k, k, idx, out, lse[0], 1.0, None, None, 0)
+    assert sfa._fwd_args(q, k, k, idx, out, lse, 1e300, None, None, 0).scale == float("inf")

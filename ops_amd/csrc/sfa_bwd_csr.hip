@@ -703,6 +703,60 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
 }
 
 // ---- 3. chunk partials -> bf16 gradients (chunk order) ----------------------
+// d = 64: gradient of key row (b, g, key) at dim `lane` from the pairs that
+// select it alone, in fp32.  The key-major products also run over unselected
+// pairs, and 0 x (a NaN or inf of q / dO) is NaN; the atomic scheme these
+// shapes had reads selected pairs only, so a result that is not finite is
+// computed again here.  want_k: dK, want_v: dV (both: their sum).  One wave; a
+// lane takes a head for P and dS and a dim for the sums.  (On finite
+// rows the forward and backward at S = 4096, 64 heads on 1, top-k 1024 take
+// 0.67 ms, as without this; its registers, 86 against 42, do not matter.)
+__device__ __forceinline__ float dkv_row64(const Params& p, int b, int g, int key, bool want_k, bool want_v) {
+  const int lane = threadIdx.x & 63;
+  const bf16* kr = reinterpret_cast<const bf16*>(p.k) + b * p.k_sb + (int64_t)key * p.k_ss + g * p.k_sh;
+  const bf16* vr = reinterpret_cast<const bf16*>(p.v) + b * p.v_sb + (int64_t)key * p.v_ss + g * p.v_sh;
+  const uint32_t* map = p.kmap + ((int64_t)b * p.Hkv + g) * p.Sq * p.kmap_w + (key >> 5);
+  const float kl = (float)kr[lane], vl = (float)vr[lane];
+  auto from_lane = [](float x, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l)); };
+  float acc = 0.f;
+  for (int t0 = 0; t0 < p.Sq; t0 += 64) {
+    const int tl = t0 + lane;
+    uint64_t sel = __ballot(tl < p.Sq && ((map[(int64_t)min(tl, p.Sq - 1) * p.kmap_w] >> (key & 31)) & 1u));
+    while (sel) {
+      const int t = t0 + __ffsll((unsigned long long)sel) - 1;
+      sel &= sel - 1;
+      for (int h0 = 0; h0 < p.G; h0 += 64) {
+        const int nh = min(64, p.G - h0), h = g * p.G + h0 + min(lane, nh - 1);
+        const bf16* qr = reinterpret_cast<const bf16*>(p.q) + b * p.q_sb + t * p.q_ss + (int64_t)h * p.q_sh;
+        const bf16* dr = reinterpret_cast<const bf16*>(p.dout) + b * p.do_sb + t * p.do_ss + (int64_t)h * p.do_sh;
+        float s = 0.f, dp = 0.f;
+#pragma unroll 1
+        for (int d = 0; d < 64; d += 8) {
+          const bf16x8 x = *reinterpret_cast<const bf16x8*>(qr + d), y = *reinterpret_cast<const bf16x8*>(dr + d);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            s += (float)x[e] * from_lane(kl, d + e);
+            dp += (float)y[e] * from_lane(vl, d + e);
+          }
+        }
+        const float lse = p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh];
+        // (lse = -inf: P = 0, but NaN where the score is; as in the query-major kernels)
+        const bool on = lse != kNegInf;
+        const float pr = exp2f(s * p.scale_log2 - (on ? lse * kLog2e : __builtin_huge_valf()));
+        const float ds = p.scale * (pr * (dp - (on ? p.delta[((int64_t)b * p.Sq + t) * p.Hq + h] : 0.f)));
+        for (int r = 0; r < nh; ++r) {
+          const int64_t hr = g * p.G + h0 + r;
+          if (want_k)
+            acc += from_lane(ds, r) * (float)(reinterpret_cast<const bf16*>(p.q) + b * p.q_sb + t * p.q_ss + hr * p.q_sh)[lane];
+          if (want_v)
+            acc += from_lane(pr, r) * (float)(reinterpret_cast<const bf16*>(p.dout) + b * p.do_sb + t * p.do_ss + hr * p.do_sh)[lane];
+        }
+      }
+    }
+  }
+  return acc;
+}
+
 // Four lanes share 4 dims of a key: lane group u of the wave sums the chunks u,
 // u + 4, ... that wrote a partial (one lane walking all of up to 64 chunks was
 // latency-bound: 44 us for 134 MB), the four sums are added in a fixed tree,
@@ -739,8 +793,19 @@ __global__ __launch_bounds__(256) void dkv_finish_kernel(Params p, GradOut out, 
         acc[e] += __shfl_xor(acc[e], o, 64);
         if constexpr (MERGE) accv[e] += __shfl_xor(accv[e], o, 64);
       }
-    if (sub != 0) continue;
     const bool is_v = !MERGE && 4 * q4 >= D;
+    if constexpr (D == 64) {  // (the wave's 16 quads are one key's dK, dV or merged row)
+      bool bad = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[e] + accv[e]) <= 3.402823466e38f);
+      if (__any(bad)) {
+        const float x = dkv_row64(p, b, g, key, MERGE || !is_v, MERGE || is_v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = __shfl(x, 4 * (lane & 15) + e, 64);
+        accv = f32x4{};
+      }
+    }
+    if (sub != 0) continue;
     const int d = is_v ? 4 * q4 - D : 4 * q4;
     if (repeats) {
       const int64_t row = (((int64_t)b * p.Skv + key) * p.Hkv + g) * D + d;

@@ -67,6 +67,27 @@ def test_repeated_keys_and_unread_rows():
         assert bool(torch.isfinite(x).all()) and _rel(x, y) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("G,Hkv,shared", [(16, 2, False), (64, 1, True), (1, 8, False)])
+def test_rows_that_are_not_finite_reach_selected_keys_only(G, Hkv, shared):
+    """Queries that select nothing may hold anything, and a NaN row reaches the
+    keys that it selects and no others."""
+    q, k, v, do, idx = _inputs(2, 1024, 1024, G, Hkv, 300, seed=4)
+    if shared:
+        v = k
+    idx[0, 100:110] = -1
+    q[0, 100:105] = float("nan")
+    do[0, 103:110] = float("inf")
+    q[1, 7, G - 1] = float("nan")  # one head of one kv head
+    do[0, 640, 0, 5] = float("nan")
+    out, lse = ops_amd.sfa_forward(q, k, v, idx)
+    a = ops_amd.sfa_backward(q, k, v, idx, out, lse, do)[:3]
+    b = ops_amd.sfa_backward(q, k, v, idx, out, lse, do, dkv_mode="atomic")[:3]
+    for x, y in zip(a, b):
+        ok = torch.isfinite(x)
+        assert torch.equal(ok, torch.isfinite(y))
+        assert _rel(torch.where(ok, x, 0.0), torch.where(ok, y, 0.0)) < 2.0 ** -8
+
+
 def test_named_scheme_stays_refused():
     q, k, v, do, idx = _inputs(1, 256, 256, 16, 1, 64, seed=3)
     out, lse = ops_amd.sfa_forward(q, k, v, idx)

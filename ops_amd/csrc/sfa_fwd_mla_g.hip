@@ -403,7 +403,11 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
 }
 
 // Merge of the fp32 split partials: one wave per row, lane s holds split s's
-// weight, a lane's 8 dims of up to 8 splits are loaded together.
+// weight, a lane's 8 dims of up to 8 splits are loaded together.  A split whose
+// sum is not a number says so in its log-sum-exp: the row's weights, and with
+// them the row, are then NaN whatever the other splits hold (a max drops a NaN,
+// so it is looked at itself).  A sink that is not finite only takes the sum: it
+// leaves zeros, as in the unsplit kernel.
 __global__ __launch_bounds__(256) void combine_f32_kernel(Params p) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t nrows = (int64_t)p.B * p.Sq * p.Hq;
@@ -428,10 +432,11 @@ __global__ __launch_bounds__(256) void combine_f32_kernel(Params p) {
   const float ls = lane < p.num_splits ? p.part_lse[lane * nrows + row] : kNegInf;
   const float sink2 = p.sink ? p.sink[h] * kLog2e : kNegInf;
   const float mm = fmaxf(wave_max(ls), sink2);
-  const float e = (ls == kNegInf || mm == kNegInf) ? 0.f : exp2f(ls - mm);
-  float l = wave_sum(e);
+  const float e = ls != ls ? ls : (ls == kNegInf || mm == kNegInf) ? 0.f : exp2f(ls - mm);
+  const float le = wave_sum(e);
+  float l = le;
   if (p.sink && mm != kNegInf) l += exp2f(sink2 - mm);
-  const float wl = l > 0.f ? e / l : (l != l ? l : 0.f);  // weight of split `lane`
+  const float wl = l > 0.f ? e / l : (le != le ? le : 0.f);  // weight of split `lane`
   f32x4 a0{}, a1{};
   for (int s0 = 0; s0 < p.num_splits; s0 += U) {
 #pragma unroll

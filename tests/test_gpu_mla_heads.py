@@ -87,6 +87,40 @@ def test_infinite_rows(splits):
     assert bool(torch.isnan(out[:, :, 1::2]).all())
 
 
+@pytest.mark.parametrize("sink", [None, 0.5, float("nan"), float("inf")])
+@pytest.mark.parametrize("what", ["nan query", "inf query", "nan cache", "one nan key"])
+@pytest.mark.parametrize("Hq", [16, 40, 128])
+def test_rows_that_are_not_numbers_survive_the_merge(Hq, what, sink):
+    """Whatever the split count, a row is NaN where the unsplit call's is, and
+    has its log-sum-exp: also when no split has a finite sum (a NaN or infinite
+    query, a cache of NaN).  (128 heads: 4 queries, the most that take this
+    kernel.)"""
+    q, kv, idx, _ = _inputs(2, 2, 300, Hq, 1, 200, seed=Hq)
+    idx[0, 0, 0] = torch.arange(200, device=DEV)
+    if what == "nan query":
+        q[0, 1, 3, 575] = float("nan")
+        q[1, 0, Hq - 1] = float("nan")
+    elif what == "inf query":
+        q[0, 1, 3, 575] = float("inf")
+    elif what == "nan cache":
+        kv[1] = float("nan")
+    else:
+        kv[0, 7, 0, 0] = float("nan")
+    s = None if sink is None else torch.full((Hq,), sink, device=DEV)
+    call = lambda n: ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, attn_sink=s, num_splits=n)
+    o_ref, l_ref = call(1)
+    bad = torch.isnan(o_ref).any(-1)
+    assert bool(bad.any()) and bool((l_ref[bad] == float("-inf")).all())
+    for n in (0, 3, 64):
+        out, lse = call(n)
+        assert torch.equal(torch.isnan(out), torch.isnan(o_ref)), n
+        ok = torch.isfinite(o_ref)
+        assert float((out.float() - o_ref.float())[ok].abs().max()) <= 2.0 ** -7 * float(o_ref[ok].float().abs().max()), n
+        assert torch.equal(torch.isfinite(lse), torch.isfinite(l_ref)) and not bool(torch.isnan(lse).any()), n
+        fin = torch.isfinite(l_ref)
+        assert not bool(fin.any()) or float((lse - l_ref)[fin].abs().max()) <= 1e-4, n
+
+
 def test_noalloc_splits_to_its_scratch():
     """The static scratch bounds the split count instead of refusing the call."""
     q, kv, idx, _ = _inputs(2, 100, 500, 64, 1, 300, seed=5)

@@ -20,10 +20,12 @@
 //    slots, conflict free); every wave forms the whole tile's softmax (the
 //    same values in each) and P^T in the B-operand layout;
 //  * O^T = V^T P^T is divided by dims, 128 per wave (32 NG accumulators).
-// P is kept to about 17 bits, as a bf16 head and a bf16 rest (two MFMAs per
-// operand), and split-k partials are fp32: the scalar kernel that these shapes
-// ran on held both in fp32, and the result's error against float64 is the same
-// (it is the output's rounding, 1.7e-3).
+// P keeps its 24 bits, as three bf16 terms (three MFMAs per operand), and
+// split-k partials are fp32: the scalar kernel that these shapes ran on held
+// both in fp32.  Share of outputs that are not the bf16 value nearest to the
+// float64 result, over prefills and decodes of 16 to 64 heads: 1.8e-4 to 3.0e-4
+// (scalar kernel 1.7e-4 to 5.5e-4; with two terms 1.7e-3 to 2.3e-3, at 450
+// against 485 us for 2048 queries of 16 heads, 1110 against 1290 us of 64).
 // Bound: the gather with 16 heads (9.1 TB/s from the Infinity Cache of the
 // 11 TB/s that whole rows reach there; 11.4 TB/s on ascending index rows, part
 // of it from L2), the matrix cores with 64.  2048 queries on 16384 keys, top-k
@@ -47,6 +49,21 @@ constexpr int kKeys = 32;             // keys per tile
 constexpr int kHalf = 256;            // slots per half of the staged index ring
 constexpr int kOT = kDv / 4 / 16;     // 16-dim O^T tiles per wave
 constexpr float kSlack = 8.0f;        // lazy-rescale slack (base-2 units)
+
+// Base-2 log-sum-exp of 2^m2 l.  The logarithm is taken of l's mantissa: that of
+// l itself, ~11 for 2048 slots below a lazy maximum, carries the rounding of
+// its whole part (relative error of the LSE against float64 6e-8, now 4e-8).
+__device__ __forceinline__ float lse2_of(float m2, float l) {
+  int e;
+  const float f = frexpf(l, &e);
+  return m2 + ((float)e + log2f(f));
+}
+// ... and the natural one
+__device__ __forceinline__ float lse_of(float m2, float l) {
+  int e;
+  const float f = frexpf(l, &e);
+  return fmaf(m2, kLn2, fmaf((float)e, kLn2, logf(f)));
+}
 
 // LDS-only barrier: the DMA in flight (vmcnt) is not waited for.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -224,8 +241,9 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
     }
     // Operand reads are issued a phase ahead of their use (the scheduling
     // barriers keep them there): ids and K operands before the next gather's
-    // address arithmetic, V^T operands before the softmax (32 heads: half of
-    // them, the registers' limit).  With each read next to its MFMA a tile of
+    // address arithmetic, V^T operands before the softmax (32 heads: two of
+    // them, paged one: more spill, 1590 and 1875 against 1455 us for paged
+    // prefills of 64 heads with two and four).  With each read next to its MFMA a tile of
     // 16 heads took 1.4 us, now 1.28.
     int raw[RG::RPW];
     if (j + 1 < ntiles) fetch_ids(j + 1, raw);
@@ -261,7 +279,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
       x[0][0] += s_x[2][lane];
       x[0][1] += s_x[3][lane];
     }
-    constexpr int PRE = NG == 1 ? kOT : kOT / 2;
+    constexpr int PRE = NG == 1 ? kOT : PAGED ? 1 : 2;
     bf16x4 vo[kOT][2];
     auto read_v = [&](int ot) {
       const uint32_t off = va[ot & 3] + (uint32_t)(ot >> 2) * 128u;
@@ -273,7 +291,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
     __builtin_amdgcn_sched_barrier(0);
 
     // softmax of head group n over this lane's 8 keys: key(kt, e) = 16 kt + 4 hq + e
-    bf16x8 phi[NG], plo[NG];
+    bf16x8 phi[NG], pmid[NG], plo[NG];
 #pragma unroll
     for (int n = 0; n < NG; ++n) {
       float sv[8];
@@ -301,7 +319,9 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
       for (int i = 0; i < 8; ++i) {
         ex[i] = __builtin_amdgcn_exp2f(sv[i] - moff);
         phi[n][i] = (bf16)ex[i];
-        plo[n][i] = (bf16)(ex[i] - (float)phi[n][i]);
+        const float rest = ex[i] - (float)phi[n][i];
+        pmid[n][i] = (bf16)rest;
+        plo[n][i] = (bf16)(rest - (float)pmid[n][i]);
       }
       l_part[n] += ((ex[0] + ex[1]) + (ex[2] + ex[3])) + ((ex[4] + ex[5]) + (ex[6] + ex[7]));
     }
@@ -315,6 +335,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
 #pragma unroll
       for (int n = 0; n < NG; ++n) {
         oacc[n][ot] = M::mma(a, phi[n], oacc[n][ot]);
+        oacc[n][ot] = M::mma(a, pmid[n], oacc[n][ot]);
         oacc[n][ot] = M::mma(a, plo[n], oacc[n][ot]);
       }
     }
@@ -338,10 +359,10 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
     const int h = g * p.G + hg0 + hl;
     const int64_t row = ((int64_t)b * p.Sq + t) * p.Hq + h;
     const float m_fin = m_used[n];
-    float scale_o, lse2;
+    float scale_o, lse;  // lse: base 2 in a partial
     if (partial) {
       scale_o = l_sum > 0.f ? 1.f / l_sum : 0.f;
-      lse2 = l_sum > 0.f ? m_fin + log2f(l_sum) : kNegInf;
+      lse = l_sum > 0.f ? lse2_of(m_fin, l_sum) : kNegInf;
     } else {
       const float sink2 = p.sink ? p.sink[h] * kLog2e : kNegInf;
       const float mm = fmaxf(m_fin, sink2);
@@ -349,13 +370,13 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
       float l = l_sum * fo;
       if (p.sink && mm != kNegInf) l += exp2f(sink2 - mm);
       scale_o = l > 0.f ? fo / l : 0.f;
-      lse2 = l > 0.f ? mm + log2f(l) : kNegInf;
+      lse = l > 0.f ? lse_of(mm, l) : kNegInf;
     }
     if (wave == 0 && hq == 0) {
       if (partial)
-        p.part_lse[split * nrows + row] = lse2;
+        p.part_lse[split * nrows + row] = lse;
       else
-        p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh] = lse2 * kLn2;
+        p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh] = lse;
     }
     nan |= l_sum != l_sum;
     // C layout: head lt, dims 128 wave + 16 ot + 4 hq + e
@@ -451,7 +472,7 @@ __global__ __launch_bounds__(256) void combine_f32_kernel(Params p) {
   }
   const bf16x8 o = {(bf16)a0[0], (bf16)a0[1], (bf16)a0[2], (bf16)a0[3], (bf16)a1[0], (bf16)a1[1], (bf16)a1[2], (bf16)a1[3]};
   *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(p.out) + b * p.o_sb + t * p.o_ss + (int64_t)h * p.o_sh + 8 * lane) = o;
-  if (lane == 0) p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh] = (l > 0.f) ? (mm + log2f(l)) * kLn2 : kNegInf;
+  if (lane == 0) p.lse[b * p.l_sb + t * p.l_ss + (int64_t)h * p.l_sh] = (l > 0.f) ? lse_of(mm, l) : kNegInf;
 }
 
 template <int NG>

@@ -181,13 +181,20 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SI
       // decode-like: too few work items to fill the chip -> split the top-k set
       splits = (int)((kTargetWorkgroups / 2 + items - 1) / items);
       // (the 128-head kernel: one workgroup per CU, so one round of at most 256,
-      // and at most 8 splits: more load Q (147 KB each) and write and merge
-      // partials longer than their tiles take.  Top-k 2048, us per call by
-      // splits: 8 sequences 32 -> 38.4, 8 -> 27.6; 16: 16 -> 34.6, 8 -> 31.1;
-      // 24: 11 -> 54.4, 8 -> 35.8; 64: 8 -> 77.9, 4 -> 65.8)
+      // and 256 slots or more a split, but up to 8 in any case: shorter ones load
+      // Q (147 KB each) and write and merge partials longer than their tiles
+      // take.  us per call by splits:
+      //   top-k  2048,  8 sequences:  4 38.5,  8  28.6, 16  33.1, 32 38.5
+      //                24 sequences:  4 41.5,  8  34.9, 10  36.6, 16 52.8
+      //   top-k  4096,  8 sequences:  8 39.3, 16  35.1, 32  38.5
+      //   top-k  8192,  8 sequences:  8 60.9, 16  46.5, 21  44.4, 32 45.7
+      //                16 sequences:  8 66.6, 10  61.0, 16  59.4, 21 82.2
+      //   top-k 16384,  8 sequences:  8 104, 16  68.5, 21  62.2, 32 62.4, 51 84.4
+      //                64 sequences:  2 313,  4 315,  8  311)
       if (sfa::fwd_mla_supported(p) && items <= kTargetWorkgroups / 4) {
+        const int cap = a->topk > 8 * 256 ? a->topk / 256 : 8;
         splits = (int)(kTargetWorkgroups / 2 / items);
-        if (splits > 8) splits = 8;
+        if (splits > cap) splits = cap;
       }
       // (the kernel for few heads: at least 4 tiles a split.  Measured at
       // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 33.7 / 23.3 /

@@ -878,10 +878,18 @@ bool mla_supported(const Params& p) {
 // 128-head kernel's 32-head waves would idle and its 256 accumulator
 // registers hold one wave per SIMD, so these have their own kernel.
 bool fwd_mla_g_supported(const Params& p) {
-  // (128 heads, top-k 2048, us per call at 16 head groups / 8 splits of the
-  // 128-head kernel: 1 sequence 20.6 / 26.6, 4 sequences 25.1 / 28.0, 8
-  // sequences 32.3 / 27.6)
-  const bool few = (int64_t)p.B * p.Sq * p.Hkv <= 4;
+  // 65 to 128 heads: a few queries, whose rows each group of 16 heads gathers
+  // again, so no more of them than the gathers stay short.  us per call, this
+  // kernel / the 128-head one, 128 heads:
+  //   queries      1          2          3          4          5
+  //   top-k 1024  18.8/21.4  18.7/21.8  19.2/22.4  19.8/23.2  24.2/23.4
+  //         2048  18.8/26.7  20.8/27.1  24.1/27.8  25.1/28.1  31.7/28.6
+  //         4096  22.5/32.9  25.8/33.0  31.6/34.7  35.3/34.9  45.7/35.0
+  //         6144  25.0/35.5  30.8/37.2  40.1/38.7  45.8/38.0
+  //         8192  27.1/38.5  36.3/40.5  47.7/40.5  59.0/42.0
+  //        12288  32.2/45.7  46.1/45.5  84.4/47.8
+  const int64_t queries = (int64_t)p.B * p.Sq * p.Hkv;
+  const bool few = queries <= 4 && queries * p.topk <= 4 * 4096;
   return p.Dqk == 576 && p.Dv == 512 && (p.G <= 64 || (p.G <= 128 && few)) && p.topk <= kMlaGMaxTopk &&
          v_is_k_prefix(p) && rows_fit_32bit(p);
 }

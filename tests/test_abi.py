@@ -129,6 +129,21 @@ def _mla_prefill_args(S, K, Skv=None):
     return a
 
 
+@pytest.mark.parametrize("B,K,splits,f32", [
+    (8, 2048, 8, False), (64, 2048, 4, False), (8, 8192, 32, False), (16, 8192, 16, False), (5, 16384, 47, False),  # (51 of 322 slots: 11 tiles of 32 each)
+    (8, 4096, 16, False), (3, 8192, 32, False), (4, 16384, 64, False), (4, 2048, 8, True), (2, 8192, 16, True),
+    (1, 12288, 32, True)])
+def test_decode_splits_grow_with_the_top_k(B, K, splits, f32):
+    """128 heads: a split keeps 256 slots or more where that leaves more than 8
+    splits, within one workgroup per CU (bf16 partials); up to 4 queries and
+    16384 slots in all take the kernel with fp32 partials."""
+    a = _mla_prefill_args(1, K, Skv=65536)
+    a.B, a.q_sb, a.o_sb, a.i_sb = B, 128 * 576, 128 * 512, K
+    ws = _lib.load().sfa_fwd_workspace_size(ctypes.byref(a))
+    rows = B * 128
+    assert ws == splits * rows * 512 * (4 if f32 else 2) + (splits * rows * 4 + 255) // 256 * 256
+
+
 def test_persistent_prefill_workspace_holds_sorted_index_rows():
     """The persistent MLA prefill (>= 4096 work items) takes 256 bytes of
     claim counters plus its index rows in ascending order (B*Sq*Hkv*topk

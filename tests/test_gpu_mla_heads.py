@@ -175,6 +175,17 @@ def test_few_queries_and_default_splits(B, Sq, Hq, Hkv):
     assert torch.equal(torch.isfinite(lse.cpu()), fin) and float((lse.cpu() - l_ref)[fin].abs().max()) < 1e-3
 
 
+# (more than 8 splits of the 128-head kernel's own choice: a long top-k, also for a few queries)
+@pytest.mark.parametrize("B,K", [(5, 4200), (2, 8448), (9, 6145)])
+def test_long_top_k_splits(B, K):
+    q, kv, idx, lens = _inputs(B, 1, 2000, 128, 1, K, seed=K)
+    idx[0, 0, 0] = torch.arange(K, device=DEV)
+    out, lse = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, kv_lens=lens)
+    o_ref, l_ref = ref_forward(q.cpu(), kv.cpu(), kv[..., :512].cpu(), idx.cpu(), 0.05, kv_lens=lens.cpu())
+    assert float((out.float().cpu() - o_ref).norm() / o_ref.norm()) < 2.0 ** -7  # (P and partials in bf16, as above)
+    assert float((lse.cpu() - l_ref).abs().max()) < 1e-3
+
+
 @pytest.mark.parametrize("G,Sq", [(16, 1301), (24, 1024), (40, 1301)])
 def test_many_queries(G, Sq):
     """Unsplit items placed in runs of 32 queries, then by eights, then singly

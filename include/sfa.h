@@ -60,9 +60,10 @@ enum {
                           <= 128, top-k <= 2048, Skv <= 262144) and cheaper: Skv <=
                           64 * top-k and CSR workspace (bitmap, lists, fp32 partials,
                           Skv * Sq * G / 16 bytes per batch and kv head and more, up to 1 GiB, in small calls)
-                          <= 4 GiB; the same scheme at d_qk = d_v = 64 when Skv <=
-                          32 * top-k and the call is large enough to repay its extra
-                          launches; otherwise ATOMIC                                       */
+                          <= 4 GiB; the same scheme at d_qk = d_v = 64 when Skv -
+                          min(Sq, Skv) / 2 <= 16 * top-k and the call is large enough
+                          (Sq * top-k * ceil(G / 16) >= 32 * Skv, and B * Hkv of those
+                          >= 2^18) to repay its extra launches; otherwise ATOMIC          */
   SFA_DKV_ATOMIC = 1,  /* fp32 atomic adds into a workspace accumulator (SFA.py:853)    */
   SFA_DKV_CSR = 2      /* deterministic: membership bitmap inverted into per-key-block
                           lists of referencing query blocks, key-major recompute, fixed-

@@ -422,8 +422,19 @@ constexpr int64_t kCsrMaxKeysPerTopk = 64;        // Skv <= 64 * top-k (<= ~32x 
 // heads, top-k 256 (32 keys per slot) 0.50 against 0.88 ms, top-k 128 (64) 0.48
 // against 0.48 ms; and enough (slot, 16 heads) pairs to repay the scheme's
 // extra launches: S = 1024, 16 heads, top-k 256 (2^18 pairs) 99 against 131 us,
-// top-k 128 (2^17) 96 against 86 us.
-constexpr int64_t kCsr64MaxKeysPerTopk = 32;
+// top-k 128 (2^17) 96 against 86 us.  Those are causal: a query sees half the
+// keys.  Queries behind a long prefix see nearly all, so the keys that a query
+// sees on average count, 16 per slot, and a key's references have to repay its
+// partials: 32 (slot, 16 heads) pairs a key.  us, key-major against atomics:
+//   128 queries,  16 heads, top-k 2048 on 65536 keys (32 a slot)  302 / 165
+//   512           16              1024    32768      (32)         390 / 251
+//   512           64               256     8192      (31)         325 / 264
+//   128           16              2048    16384 ( 8; 16 a key)    153 / 143
+//   128           16              2048     8192 ( 4; 32 a key)    141 / 140
+//   512           16              2048    32768 (16; 32 a key)    428 / 454
+//   512           32               256     4096 (15; 64 a key)    110 / 140
+constexpr int64_t kCsr64MaxSeenPerTopk = 16;
+constexpr int64_t kCsr64MinPairsPerKey = 32;
 constexpr int64_t kCsr64MinSlots = int64_t(1) << 18;
 constexpr size_t kCsrMaxWorkspace = size_t(4) << 30;  // CSR arrays + partials <= 4 GiB
 
@@ -440,8 +451,14 @@ bool use_csr(const sfa_bwd_args* a, sfa::Params p) {
   if (!(bwd_mfma_ok(a) && sfa::bwd_csr_supported(p) && sfa::bwd_dq_supported(p))) return false;
   // (asked for by name it is the d = 128 scheme, as its contract says)
   if (a->dkv_mode == SFA_DKV_CSR) return p.Dqk == 128;
-  if ((int64_t)p.Skv > (p.Dqk == 64 ? kCsr64MaxKeysPerTopk : kCsrMaxKeysPerTopk) * p.topk) return false;
-  if (p.Dqk == 64 && (int64_t)p.B * p.Sq * p.Hkv * p.topk * ((p.G + 15) / 16) < kCsr64MinSlots) return false;
+  if (p.Dqk == 64) {
+    const int64_t pairs = (int64_t)p.Sq * p.topk * ((p.G + 15) / 16);  // of a (batch, kv head)
+    const int64_t seen2 = 2 * (int64_t)p.Skv - (p.Sq < p.Skv ? p.Sq : p.Skv);  // twice the keys a causal query sees
+    if (seen2 > 2 * kCsr64MaxSeenPerTopk * p.topk || pairs < kCsr64MinPairsPerKey * p.Skv) return false;
+    if (p.B * p.Hkv * pairs < kCsr64MinSlots) return false;
+  } else if ((int64_t)p.Skv > kCsrMaxKeysPerTopk * p.topk) {
+    return false;
+  }
   sfa::csr_geometry(p);
   return sfa::csr_workspace_bytes(p) <= kCsrMaxWorkspace;
 }

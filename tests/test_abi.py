@@ -144,6 +144,33 @@ def test_decode_splits_grow_with_the_top_k(B, K, splits, f32):
     assert ws == splits * rows * 512 * (4 if f32 else 2) + (splits * rows * 4 + 255) // 256 * 256
 
 
+@pytest.mark.parametrize("Sq,Skv,G,Hkv,K,keymajor", [
+    (4096, 4096, 64, 1, 1024, True), (8192, 8192, 16, 1, 256, True), (8192, 8192, 16, 1, 255, False),
+    (1024, 1024, 16, 1, 256, True), (1024, 1024, 16, 1, 255, False), (1024, 1024, 1, 16, 64, True),
+    (512, 32768, 16, 1, 2048, True), (128, 8192, 16, 1, 2048, True), (128, 65536, 16, 1, 2048, False),
+    (512, 32768, 16, 1, 1024, False), (128, 16384, 16, 1, 2048, False), (512, 8192, 64, 1, 256, False)])
+def test_d64_backward_scheme_follows_the_keys_a_query_sees(Sq, Skv, G, Hkv, K, keymajor):
+    """d = 64 under AUTO: key-major where the call is large, a query sees at
+    most 16 keys a slot (causally) and a key has 32 (slot, 16 heads) pairs;
+    the fp32 atomics, whose workspace has no bitmap, elsewhere."""
+    lib = _lib.load()
+    b = _lib.BwdArgs()
+    a = b.fwd = _valid_args()
+    Hq = G * Hkv
+    a.B, a.Sq, a.Skv, a.Hq, a.Hkv, a.Dqk, a.Dv, a.topk = 1, Sq, Skv, Hq, Hkv, 64, 64, K
+    a.k_sh = a.v_sh = a.q_sh = a.o_sh = b.do_sh = b.dq_sh = b.dk_sh = b.dv_sh = 64
+    a.k_ss = a.v_ss = b.dk_ss = b.dv_ss = Hkv * 64
+    a.q_ss = a.o_ss = b.do_ss = b.dq_ss = Hq * 64
+    a.l_sh, a.l_ss, a.l_sb = 1, Hq, Sq * Hq
+    a.i_sh, a.i_ss, a.i_sb = K, Hkv * K, Sq * Hkv * K
+    for name in ("dout", "dq", "dk", "dv"):
+        setattr(b, name, 0x10000)
+    b.fwd, b.dkv_mode = a, 1
+    atomic = lib.sfa_bwd_workspace_size(ctypes.byref(b))
+    b.dkv_mode = 0
+    assert (lib.sfa_bwd_workspace_size(ctypes.byref(b)) > atomic) == keymajor and atomic > 0
+
+
 def test_persistent_prefill_workspace_holds_sorted_index_rows():
     """The persistent MLA prefill (>= 4096 work items) takes 256 bytes of
     claim counters plus its index rows in ascending order (B*Sq*Hkv*topk

@@ -98,22 +98,6 @@ __device__ __forceinline__ int bound_of(const Params& p, int b) {
   return n < p.Skv ? n : p.Skv;
 }
 
-// Workgroup id -> work item ((b Sq + t) Hkv + g) of a launch of one workgroup
-// per item.  Workgroups go to the 8 XCDs in turn (id % 8), each with a 4 MB L2:
-//  * with 2, 4 or 8 kv heads an XCD works on one of them, so that its L2
-//    holds that head's rows only;
-//  * the XCDs of a head get runs of 32 consecutive queries in turn, whose
-//    common keys (a recency window) meet in L2; queries that do not fill a
-//    round of runs follow one by one.
-__device__ __forceinline__ int xcd_item(const Params& p, int id) {
-  const int lh = p.Hkv == 8 ? 3 : p.Hkv == 4 ? 2 : p.Hkv == 2 ? 1 : 0;  // log2 of the heads told apart
-  const int nq = (int)((unsigned)p.B * p.Sq * p.Hkv >> lh);
-  const int runs = nq & -(256 >> lh);  // queries in runs (a round: 32 on each of a head's 8 >> lh XCDs)
-  if (id >= runs << lh) return id;
-  const int x = id & 7, r = id >> 3;
-  return (((((r >> 5) << (3 - lh)) + (x >> lh)) << 5) + (r & 31) << lh) + (x & ((1 << lh) - 1));
-}
-
 // Pool row (page * page_size + offset) of logical key id of sequence b in
 // paged mode, or -1 when the slot is invalid (id outside [0, bound)) or its
 // page is unmapped (block-table entry outside [0, num_pages)).

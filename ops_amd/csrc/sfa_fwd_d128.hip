@@ -77,7 +77,14 @@ __global__ __launch_bounds__(64, 3) void fwd_d128_kernel(Params p) {
 
   // ---- work item (same placement as the MLA kernel) ----------------------
   // A sub-item is (split, head group): the sub-items of one item go to the
-  // same XCD, so its L2 serves them the item's rows.
+  // same XCD, so its L2 serves them the item's rows.  Items of one sub-item
+  // are taken in order: with 2, 4 or 8 kv heads an XCD (workgroup id % 8) then
+  // works on one of them, with more on an eighth of them, and its 4 MB L2
+  // holds those heads' rows only.  Runs of 32 queries per XCD, whose recent
+  // keys would meet in L2, gave nothing on top with 1 to 8 heads (B = 2, S =
+  // 8192, 2 heads: 716 and 717 us) and put every head on every XCD with more
+  // (4096 queries, top-k 512, 12 / 16 / 32 heads: 1037 / 1504 / 3594 us, in
+  // order 532 / 645 / 1639).
   int wi = blockIdx.x;
   const int nhs = (p.G + kT - 1) / kT;  // head groups of 16
   const int nsub = p.num_splits * nhs;
@@ -87,9 +94,6 @@ __global__ __launch_bounds__(64, 3) void fwd_d128_kernel(Params p) {
     const int x = wi % 8, r = wi / 8;
     sub = r % nsub;
     wi = (r / nsub) * 8 + x;
-  } else if (nsub == 1) {
-    sub = 0;
-    wi = xcd_item(p, wi);
   } else {
     sub = wi % nsub;
     wi /= nsub;

@@ -198,31 +198,15 @@ __global__ __launch_bounds__(256) void csr_scatter_wave_kernel(Params p) {
 // key-major kernel.  One workgroup: a unit's position is its class's start
 // plus the count of earlier units of its class (ballots, then a prefix over
 // the waves of the tile and the tiles before it).
-// One list per (b, g), up to 8 (then (b, g) mod 8): XCD x claims from list x
-// mod lists, so that the units running on it read one (b, g)'s query blocks
-// (4 MB of Q and dO per chunk of 64 blocks: an XCD's L2) and from the others
-// once that is exhausted.  One workgroup per list.  Only in large calls (chunks
-// of 64 and up): B = 2, S = 8192, 2 kv heads 2270 -> 2195 us, but the failing
-// claims at the end of S = 2048, 8 kv heads cost the backward 30 of 360 us.
-__host__ __device__ inline int unit_lists(const Params& p) {
-  return p.chunk < 64 ? 1 : p.B * p.Hkv < 8 ? p.B * p.Hkv : 8;
-}
-__host__ __device__ inline int units_per_list(const Params& p) {
-  return (p.B * p.Hkv + unit_lists(p) - 1) / unit_lists(p) * p.nkb * p.max_chunks;
-}
 constexpr int kClasses = 8;
 __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
   __shared__ int s_cnt[16][kClasses];
   __shared__ int s_start[kClasses];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nbg = p.B * p.Hkv, per_chunk = nbg * p.nkb, nunits = per_chunk * p.max_chunks;
-  const int list = blockIdx.x, lists = unit_lists(p);
-  int* const ctr = p.kctr + 8 + 2 * list;
-  int* const order = p.uorder + (int64_t)list * units_per_list(p);
-  auto cls = [&](int u) -> int {  // class of unit u, -1 if it is another list's or has no query block
+  auto cls = [&](int u) -> int {  // class of unit u, -1 if it has no query block
     const int c = p.max_chunks - 1 - u / per_chunk;
     const int kb = (u % per_chunk) / nbg, bg = (u % per_chunk) % nbg;
-    if (bg % lists != list) return -1;
     const int* start = p.bstart + ((int64_t)bg * p.nkb + kb) * (p.max_chunks + 1);
     const int n = start[c + 1] - start[c];
     return n > 0 ? kClasses * (p.chunk - n) / p.chunk : -1;
@@ -246,8 +230,8 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
       s_start[j] = acc;
       for (int w = 0; w < 16; ++w) acc += s_cnt[w][j];
     }
-    ctr[0] = 0;
-    ctr[1] = acc;
+    p.kctr[0] = 0;
+    p.kctr[1] = acc;
   }
   __syncthreads();
   // positions, tile by tile in base order
@@ -265,7 +249,7 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
     if (k >= 0) {
       int pos = s_start[k] + rank;
       for (int w = 0; w < wave; ++w) pos += s_cnt[w][k];
-      order[pos] = u;
+      p.uorder[pos] = u;
     }
     __syncthreads();
     if (tid < kClasses) {
@@ -310,7 +294,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
   // published in the other slot behind unit i's barriers
   __shared__ int s_unit[2];
 
-  // Units are claimed in the order unit_order_kernel lists
+  // Units are claimed from one counter in the order unit_order_kernel lists
   // them (the full ones first, grouped by query range; the short ones last).
   // Claiming balances the CUs however unequal the units are (a fixed unit ->
   // workgroup mapping leaves CUs idle: workgroups are dispatched to the XCDs
@@ -321,24 +305,13 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
   // (an offset the compiler cannot prove uniform keeps the atomic a single
   // lane's: for a uniform address it is rewritten into a wave reduction that
   // waits for every load in flight)
-  // (thread 0) the list it claims from; claim_end: the unit of a claim's
-  // counter value, from the next lists once this one is exhausted
-  const int lists = unit_lists(p_arg);
-  int list = (int)(blockIdx.x % 8) % lists;
-  auto claim_start = [&](const Params& q) {
-    int o = 8 + 2 * list;
+  auto claim = [](const Params& q) {
+    int o = 0;
     asm volatile("" : "+v"(o));
-    return atomicAdd(q.kctr + o, 1);
+    const int i = atomicAdd(q.kctr + o, 1);
+    return i < q.kctr[1] ? q.uorder[i] : -1;
   };
-  auto claim_end = [&](const Params& q, int i) {
-    for (int k = 0;; ++k) {
-      if (i < q.kctr[9 + 2 * list]) return q.uorder[(int64_t)list * units_per_list(q) + i];
-      if (k + 1 >= lists) return -1;
-      list = list + 1 == lists ? 0 : list + 1;
-      i = claim_start(q);
-    }
-  };
-  if (threadIdx.x == 0) s_unit[0] = claim_end(p_arg, claim_start(p_arg));
+  if (threadIdx.x == 0) s_unit[0] = claim(p_arg);
   __syncthreads();
   int par = 0;
   for (;;) {
@@ -354,7 +327,11 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
   // the end of the unit (waiting for it here would also wait for this
   // workgroup's partial stores of the previous unit, still in flight)
   int claim_i = 0;
-  if (tid == 0) claim_i = claim_start(p);
+  if (tid == 0) {
+    int o = 0;
+    asm volatile("" : "+v"(o));
+    claim_i = atomicAdd(p.kctr + o, 1);
+  }
   const int c = p.max_chunks - 1 - u / per_chunk;
   const int kb = (u % per_chunk) / nbg;
   const int bg = (u % per_chunk) % nbg;
@@ -365,7 +342,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
   const int e0 = __builtin_amdgcn_readfirstlane(start[c]);
   const int nblk = __builtin_amdgcn_readfirstlane(start[c + 1]) - e0;
   if (nblk <= 0) {  // no query block of this chunk selects the key block
-    if (tid == 0) s_unit[par ^ 1] = claim_end(p, claim_i);
+    if (tid == 0) s_unit[par ^ 1] = claim_i < p.kctr[1] ? p.uorder[claim_i] : -1;
     par ^= 1;
     __syncthreads();
     continue;
@@ -696,7 +673,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
       *reinterpret_cast<f32x4*>(part + kD + dim) = v4;
     }
   }
-  if (tid == 0) s_unit[par ^ 1] = claim_end(p, claim_i);
+  if (tid == 0) s_unit[par ^ 1] = claim_i < p.kctr[1] ? p.uorder[claim_i] : -1;
   par ^= 1;
   __syncthreads();  // the next unit's list and blocks overwrite the LDS; its claim is published
   }  // units
@@ -883,7 +860,7 @@ size_t csr_workspace_bytes(const Params& p) {
   return al256(bg * p.Sq * p.kmap_w * 4) + al256((size_t)p.B * p.Sq * p.Hkv * p.topk) +
          al256(bg * p.nkb * p.nqb * 4) + al256(bg * p.nkb * (p.max_chunks + 1) * 4) +
          al256(bg * p.nkb * p.max_chunks * kKeyBlock * 2 * p.Dqk * 4) + al256((size_t)2 * p.B * p.Sq * p.Hq * 4) + 256 +
-         al256((size_t)unit_lists(p) * units_per_list(p) * 4);
+         al256(bg * p.nkb * p.max_chunks * 4);
 }
 
 void csr_bind_workspace(Params& p, void* ws) {
@@ -913,7 +890,7 @@ hipError_t launch_csr_index(const Params& p, hipStream_t s) {
   else
     hipLaunchKernelGGL(csr_scatter_kernel, dim3((unsigned)rows), dim3(256), 0, s, p);
   hipLaunchKernelGGL(csr_blocklist_kernel, dim3((unsigned)((int64_t)p.B * p.Hkv * p.nkb)), dim3(256), 0, s, p);
-  hipLaunchKernelGGL(unit_order_kernel, dim3((unsigned)unit_lists(p)), dim3(1024), 0, s, p);
+  hipLaunchKernelGGL(unit_order_kernel, dim3(1), dim3(1024), 0, s, p);
   return hipGetLastError();
 }
 

@@ -66,10 +66,9 @@ struct Params {
   int* bstart;        // [B][Hkv][nkb][max_chunks + 1] blist index of each 128-query-block chunk's first entry
   float* dkv_part;    // [B][Hkv][nkb][max_chunks][128][2 D] fp32 partial dK | dV per chunk
   float* rowc;        // [2][B*Sq*Hq] per row: -lse / scale, then -δ (written by the δ pass)
-  int* kctr;          // key-major claims: per list l a counter [8 + 2 l] and its listed units [9 + 2 l] (set by
-                      // unit_order_kernel); [2] nonzero if a row repeats a key (cleared by the δ pass, set by the
-                      // inversion)
-  int* uorder;        // [lists][units per list] key-major units in claim order (non-empty ones only)
+  int* kctr;          // key-major claims: [0] counter, [1] listed units (both set by unit_order_kernel);
+                      // [2] nonzero if a row repeats a key (cleared by the δ pass, set by the inversion)
+  int* uorder;        // [B*Hkv*nkb*max_chunks] key-major units in claim order (non-empty ones only)
   int nkb, nqb;       // key blocks (128 keys), query blocks (128 / G queries)
   int lg_g;           // log2(G)
   int max_chunks;     // chunks per key block (query blocks / chunk, rounded up)

@@ -16,7 +16,8 @@ DEV = "cuda"
 # (causal (key block, query block) pairs / 512: 0.3, 2.1, 5.9, 6.2, 23.8, 24.4, 192 and above; D, B, S, heads, kv heads, K)
 @pytest.mark.parametrize("D,B,S,Hq,Hkv,K", [
     (128, 1, 300, 16, 1, 96), (128, 1, 1030, 16, 1, 200), (64, 1, 1700, 16, 1, 300), (128, 1, 1790, 16, 1, 130),
-    (128, 1, 1750, 64, 1, 100), (128, 1, 1800, 128, 2, 70), (128, 1, 5025, 128, 1, 90)])
+    (128, 1, 1750, 64, 1, 100), (128, 1, 1800, 128, 2, 70), (128, 1, 5025, 128, 1, 90),
+    (128, 2, 8300, 64, 8, 130)])  # (the last: chunks of 64 blocks would take 1.2 GB of partials, so 128)
 def test_chunks(D, B, S, Hq, Hkv, K):
     g = torch.Generator(device=DEV).manual_seed(S)
     q, do = (torch.randn((B, S, Hq, D), generator=g, device=DEV).bfloat16() for _ in range(2))

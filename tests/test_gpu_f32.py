@@ -96,6 +96,35 @@ def test_infinite_rows_and_pages():
     assert _rel(got, want.cpu()) < TOL
 
 
+def test_pages_over_several_windows():
+    """More than one 256-slot window, pages in between, one page unmapped."""
+    q, k, v, _, idx, lens = _inputs(2, 5, 512, 20, 1, 128, 700, seed=8)
+    kp, vp, bt = page_kv(k, v, 16, seed=1, spare_pages=2)
+    bt[1, 4] = -1
+    drop = idx.clone()
+    drop[1][(drop[1] >= 64) & (drop[1] < 80)] = -1
+    a = ops_amd.sfa_forward(q, k, v, drop, kv_lens=lens)
+    b = ops_amd.sfa_forward_paged(q, kp, vp, bt, idx, kv_lens=lens)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    o_ref, _ = ref_forward(q.cpu(), k.cpu(), v.cpu(), drop.cpu(), kv_lens=lens.cpu(), dtype=torch.float64)
+    assert _rel(b[0], o_ref) < TOL
+
+
+@pytest.mark.parametrize("K", [8192, 8193])
+def test_longest_rows_and_beyond(K):
+    """8192 slots are the matrix kernels' longest rows, the scalar kernels take
+    8193.  (Sums of 8192 terms of random sign: sqrt(8192) * 2^-24 = 5.4e-6.)"""
+    q, k, v, do, idx, _ = _inputs(1, 2, 900, 4, 1, 64, K, seed=9)
+    idx[0, 1] = torch.arange(K, device=DEV) % 1000 - 50
+    out, lse = ops_amd.sfa_forward(q, k, v, idx)
+    c = [x.cpu() for x in (q, k, v, idx)]
+    o_ref, l_ref = ref_forward(*c, dtype=torch.float64)
+    assert _rel(out, o_ref) < TOL and _rel(lse, l_ref) < TOL
+    ref = ref_backward(*c, o_ref, l_ref, do.cpu().double(), dtype=torch.float64)
+    for x, y in zip(ops_amd.sfa_backward(q, k, v, idx, out, lse, do)[:3], ref):
+        assert _rel(x, y) < TOL
+
+
 def test_rows_without_a_finite_score_have_no_gradient():
     """A query whose only selected key scores -inf has lse = -inf: its dq is 0
     and it adds nothing to dk / dv, whatever the key's rows hold."""

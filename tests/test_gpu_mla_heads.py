@@ -211,3 +211,31 @@ def test_many_queries(G, Sq):
         assert torch.equal(out, o2) and torch.equal(lse, l2)
     o3, l3 = ops_amd.sfa_forward(q, kv, kv[..., :512], idx, 0.05, noalloc=True)
     assert torch.equal(out, o3) and torch.equal(lse, l3)
+
+
+@pytest.mark.parametrize("G,Hkv,Sq,paged", [(16, 2, 520, False), (32, 1, 1024, True), (16, 2, 600, True)])
+def test_ascending_rows_of_kv_heads_and_pages(G, Hkv, Sq, paged):
+    """The library's ascending rows with two kv heads and over pages (one of
+    them unmapped): bitwise those that the caller sorts, and on pages bitwise
+    the contiguous call's."""
+    q, kv, idx, lens = _inputs(1, Sq, 8192, G * Hkv, Hkv, 520, seed=Sq)
+    idx = torch.stack([torch.randperm(8192 + 512, device=DEV)[:520] for _ in range(Sq * Hkv)]).view(1, Sq, Hkv, 520).int()
+    call = lambda ids, **kw: ops_amd.sfa_forward(q, kv, kv[..., :512], ids, 0.05, kv_lens=lens, **kw)
+    n = int(lens[0])
+    if paged:
+        kp, vp, bt = page_kv(kv, kv[..., :512], 64, seed=2, spare_pages=5)
+        bt[0, 7] = -1
+        out, lse = ops_amd.sfa_forward_paged(q, kp, vp, bt, idx, 0.05, kv_lens=lens)
+        # (the unmapped page's slots keep their place in the ascending row: drop them there)
+        key = torch.where(idx < n, idx, 8192)
+        asc = key.sort(-1).values
+        asc = torch.where((asc >= 448) & (asc < 512), -1, torch.where(asc == 8192, -1, asc)).int()
+        ref = call(asc, idx_sorted=True)
+    else:
+        out, lse = call(idx)
+        asc = torch.where(idx < n, idx, 8192).sort(-1).values
+        ref = call(torch.where(asc == 8192, -1, asc).int(), idx_sorted=True)
+    assert torch.equal(out, ref[0]) and torch.equal(lse, ref[1])
+    o_ref, l_ref = ref_forward(q[:, ::97].cpu(), kv.cpu(), kv[..., :512].cpu(), (asc if paged else idx)[:, ::97].cpu(), 0.05,
+                               kv_lens=lens.cpu())
+    _check(out[:, ::97], lse[:, ::97], (o_ref, l_ref))

@@ -95,7 +95,7 @@ def _reads(ins: str):
     if len(parts) < 2:
         return set()
     ops = parts[1].split(",")
-    if ins.startswith(("ds_write", "global_store", "buffer_store", "flat_store")):
+    if ins.startswith(("ds_write", "global_store", "buffer_store", "flat_store", "scratch_store")):
         return set().union(*[_regs(o) for o in ops])
     return set().union(*[_regs(o) for o in ops[1:]]) if len(ops) > 1 else set()
 
@@ -140,7 +140,7 @@ def scan_result_reads(asm: str, kernels=INLINE_ASM_MFMA_KERNELS, drain: int = DR
                             hits.add(nxt)
                         if _regs(mops[0]) & dst:
                             break
-                    elif nxt.startswith(("v_", "ds_", "global_", "buffer_", "flat_")) and _reads(nxt) & dst:
+                    elif nxt.startswith(("v_", "ds_", "global_", "buffer_", "flat_", "scratch_")) and _reads(nxt) & dst:
                         hits.add(nxt)
                     waits += 1
                     if nxt.startswith("s_branch"):
@@ -193,6 +193,15 @@ def test_result_scanner_flags_a_planted_early_read():
            "\ts_nop 7\n\ts_nop 7\n\ts_nop 3\n\tv_add_f32_e32 v20, v33, v33\n.Lfunc_end0:\n")
     hits = scan_result_reads(asm)
     assert [h[2] for h in hits] == ["v_add_f32_e32 v20, v3, v3"]
+
+
+def test_result_scanner_flags_a_planted_early_spill():
+    # a spill of a result (all of a scratch store's operands are read); a
+    # reload into other registers and a spill after the drain are not reported
+    asm = ("_Zdkv_keymajor_kernel_planted:\n\tv_mfma_f32_32x32x16_bf16 v[0:15], v[16:19], v[24:27], v[0:15]\n"
+           "\tscratch_store_dwordx4 off, v[4:7], s32 offset:16\n\tscratch_load_dword v40, off, s32 offset:32\n"
+           "\ts_nop 7\n\ts_nop 7\n\ts_nop 3\n\tscratch_store_dword off, v2, s32\n.Lfunc_end0:\n")
+    assert [h[2] for h in scan_result_reads(asm)] == ["scratch_store_dwordx4 off, v[4:7], s32 offset:16"]
 
 
 def test_result_scanner_follows_branches_and_agprs():

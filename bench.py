@@ -279,7 +279,7 @@ def bench_mla_prefill(args):
 
 
 def bench_tiny(args):
-    """Config 1 (fp32, generic kernels): fwd + bwd TFLOP/s."""
+    """Config 1 (fp32): fwd + bwd TFLOP/s."""
     import ops_amd
     from ops_amd.workloads import make_workload
     w = make_workload("tiny", device="cuda")

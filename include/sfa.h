@@ -58,13 +58,15 @@ enum { SFA_DTYPE_F32 = 0, SFA_DTYPE_BF16 = 1, SFA_DTYPE_FP8_E4M3 = 2 };
 enum {
   SFA_DKV_AUTO = 0,    /* CSR where supported (bf16, d_qk = d_v = 128, G a power of two
                           <= 128, top-k <= 2048, Skv <= 262144) and cheaper: Skv <=
-                          64 * top-k and CSR workspace (bitmap, lists, fp32 partials,
-                          Skv * Sq * G / 16 bytes per batch and kv head and more, up to 1 GiB, in small calls)
+                          64 * top-k and CSR workspace (bitmap, lists, fp32 partials of
+                          8 * d bytes per key and chunk of 4 to 64 blocks of 128
+                          query-head rows, longer where those would pass 1 GiB)
                           <= 4 GiB; the same scheme at d_qk = d_v = 64 when Skv -
                           min(Sq, Skv) / 2 <= 16 * top-k and the call is large enough
                           (Sq * top-k * ceil(G / 16) >= 32 * Skv, and B * Hkv of those
                           >= 2^18) to repay its extra launches; otherwise ATOMIC          */
-  SFA_DKV_ATOMIC = 1,  /* fp32 atomic adds into a workspace accumulator (SFA.py:853)    */
+  SFA_DKV_ATOMIC = 1,  /* fp32 atomic adds (SFA.py:853) into a workspace accumulator;
+                          float32 at d_qk = d_v = 64 or 128 into dk / dv themselves    */
   SFA_DKV_CSR = 2      /* deterministic: membership bitmap inverted into per-key-block
                           lists of referencing query blocks, key-major recompute, fixed-
                           order reduction (index rows that repeat a key take atomics for

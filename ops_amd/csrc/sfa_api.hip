@@ -197,11 +197,11 @@ FwdPlan plan_fwd(const sfa_fwd_args* a, const sfa_kv_pages* pg, size_t room = SI
         if (splits > cap) splits = cap;
       }
       // (the kernel for few heads: at least 4 tiles a split.  Measured at
-      // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 33.7 / 23.3 /
-      // 20.3 us, 64 splits 38.5 / 35.2 / 24.7 us: shorter splits load more Q
+      // top-k 2048, 4 sequences, 64 / 32 / 16 heads: 16 splits 25.6 / 22.5 /
+      // 17.4 us, 64 splits 31.5 / 33.2 / 23.2 us: shorter splits load more Q
       // and write more partial rows than the idle CUs repay)
       // (two of its workgroups share a CU: a second one per CU pays while a
-      // split keeps 16 tiles; 64 sequences of 64 heads, 2 / 4 splits 82 / 67 us)
+      // split keeps 16 tiles; 64 sequences of 64 heads, 2 / 4 splits 75 / 66 us)
       if (sfa::fwd_partials_f32(p)) {
         if (a->topk >= 2 * splits * 16 * nk) splits *= 2;
         if (splits > (a->topk + 4 * nk - 1) / (4 * nk)) splits = (a->topk + 4 * nk - 1) / (4 * nk);

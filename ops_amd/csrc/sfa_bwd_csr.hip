@@ -19,20 +19,21 @@
 //     consecutive query blocks (an absolute query range) begins in it.
 //  2. Key-major recompute.  A work unit is a key block (each wave 32 keys, K
 //     and V rows kept in registers) and one chunk: the listed query blocks in
-//     one absolute range of p.chunk query blocks.  One persistent workgroup
-//     per CU claims units from a counter, longest first and otherwise in
-//     chunk-descending order, so the units that run together are key blocks
-//     of the same query range and read the same query blocks.  Per query block it recomputes, for every (row, key)
-//     pair of the block, S = Q K^T and dP = dO V^T (32x32x16 MFMA, rows as
+//     one absolute range of p.chunk query blocks.  Persistent workgroups (one
+//     per CU, two at d = 64) claim units from a counter, longest first and
+//     otherwise in chunk-descending order, so the units that run together are
+//     key blocks of the same query range and read the same query blocks.  Per
+//     query block one recomputes, for every (row, key) pair, S = Q K^T and dP = dO V^T (32x32x16 MFMA, rows as
 //     M, keys as N), P = 2^(S scale log2e - lse2) and dS = P (dP - δ) masked
 //     by the bitmap, and accumulates dV^T += dO^T P and dK^T += Q^T dS in
 //     AGPRs (the C layout of S is the B layout of these products; the A
 //     operands are transposing LDS reads of 4-row runs in the matching
-//     order).  Pairs that are not selected get P = 0, so a block costs the
+//     order; at d = 64 the accumulators fit VGPRs).  Pairs that are not selected get P = 0, so a block costs the
 //     same whatever its density.
 //  3. Reduction.  The chunks of a key block write fp32 partials; a reduction
-//     kernel adds them in chunk order and writes the bf16 gradients (no cleared
-//     accumulators, no separate conversion: those exist for repeated keys only).
+//     kernel adds them in a fixed order (every fourth chunk in a chain, the four
+//     sums as a tree) and writes the bf16 gradients (no cleared accumulators, no
+//     separate conversion: those exist for repeated keys only).
 
 #include "sfa_common.h"
 #include "sfa_lds.h"
@@ -268,8 +269,8 @@ __global__ __launch_bounds__(1024) void unit_order_kernel(Params p) {
 // reads of one are not made to wait for DMA into the other.
 // d = 64: the operands, accumulators and block buffers are half as large (70 KB
 // of LDS), so two workgroups share a CU.  S = 4096, 64 heads on one kv row,
-// top-k 1024: this kernel 0.42 ms and the whole backward 0.60-0.69 ms, against
-// 6.14 ms with fp32 atomics for every pair.
+// top-k 1024: this kernel 0.37-0.39 ms, forward and backward 0.66 ms, against
+// 6.3 ms with fp32 atomics for every pair.
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Params p_arg) {
   constexpr int kD = D;                   // head dim (d_qk = d_v)
@@ -545,7 +546,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void dkv_keymajor_kernel(Para
         const float pr = __uint_as_float(__float_as_uint(ex) & keep);
         float ds = pr * dpa[e];
         // (d = 64: the mask again, as an unselected key row may hold anything and
-        // 0 * NaN is NaN; the atomic scheme these shapes had never read it)
+        // 0 * NaN is NaN.  The reduction would recompute such a row, see
+        // dkv_row64, but rows of a cache that nothing wrote yet should not cost that)
         if constexpr (D == 64) ds = __uint_as_float(__float_as_uint(ds) & keep);
         pp[jj] = (bf16)pr;
         dd[jj] = (bf16)ds;
@@ -843,8 +845,12 @@ void csr_geometry(Params& p) {
   //     8 (S 2048, 16 on 1)              563  331  226  177  191  207
   //     4 (S 1024, 32 on 2)              544  313  202  149  130  147
   //   1.5 (S 600, 32 on 8)               187  180  179  170  144  132
-  // (d = 64 has its minima at the same places.)  Below 128 the partials stay
-  // within 1 GiB.
+  // (d = 64 has its minima at the same places.)  Calls whose queries select
+  // keys of the whole sequence have twice the pairs and even units, where long
+  // chunks lose nothing: S = 16384, 16 heads, 128 / 64: 4759 / 4937 (causal
+  // 2937 / 2871), S = 8192, 8 heads, 128 / 32: 857 / 905 (causal 836 / 690); the
+  // host cannot tell them apart, and causal ones are the rule in training.
+  // Chunks grow while the partials would pass 1 GiB.
   const int64_t bg = (int64_t)p.B * p.Hkv, pairs = bg * p.nkb * p.nqb / 2;
   p.chunk = pairs >= 192 * 256 ? 64 : pairs >= 24 * 256 ? 32 : pairs >= 6 * 256 ? 16 : pairs >= 2 * 256 ? 8 : 4;
   for (;; p.chunk *= 2) {

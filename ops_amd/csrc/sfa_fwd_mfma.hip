@@ -866,10 +866,9 @@ bool rows_fit_32bit(const Params& p) {
   return kb < (int64_t)kOOB && vb < (int64_t)kOOB && fits_u24(2 * p.k_ss) && fits_u24(2 * p.v_ss);
 }
 
-}
-namespace {
 bool mla_supported(const Params& p) {
-  return p.Dqk == 576 && p.Dv == 512 && p.G <= 128 && p.G > 64 && v_is_k_prefix(p) && rows_fit_32bit(p) && !fwd_mla_g_supported(p);
+  return p.Dqk == 576 && p.Dv == 512 && p.G <= 128 && p.G > 64 && v_is_k_prefix(p) && rows_fit_32bit(p) &&
+         !fwd_mla_g_supported(p);
 }
 
 }  // namespace
@@ -882,12 +881,12 @@ bool fwd_mla_g_supported(const Params& p) {
   // again, so no more of them than the gathers stay short.  us per call, this
   // kernel / the 128-head one, 128 heads:
   //   queries      1          2          3          4          5
-  //   top-k 1024  18.8/21.4  18.7/21.8  19.2/22.4  19.8/23.2  24.2/23.4
-  //         2048  18.8/26.7  20.8/27.1  24.1/27.8  25.1/28.1  31.7/28.6
-  //         4096  22.5/32.9  25.8/33.0  31.6/34.7  35.3/34.9  45.7/35.0
-  //         6144  25.0/35.5  30.8/37.2  40.1/38.7  45.8/38.0
-  //         8192  27.1/38.5  36.3/40.5  47.7/40.5  59.0/42.0
-  //        12288  32.2/45.7  46.1/45.5  84.4/47.8
+  //   top-k 1024  17.9/21.5  18.5/21.8  19.6/22.3  19.9/22.9  25.2/23.7
+  //         2048  19.1/26.4  21.0/27.0  24.6/27.6  25.2/28.1  33.1/28.9
+  //         4096  22.5/32.5  26.1/32.7  32.2/34.0  35.8/34.6  47.6/34.8
+  //         6144  25.1/35.0  31.3/36.8  40.9/37.7  45.9/36.8
+  //         8192  27.2/37.8  36.2/40.0  49.0/39.8  58.6/40.2
+  //        12288  32.8/44.9  46.2/45.0  86.1/45.9
   const int64_t queries = (int64_t)p.B * p.Sq * p.Hkv;
   const bool few = queries <= 4 && queries * p.topk <= 4 * 4096;
   return p.Dqk == 576 && p.Dv == 512 && (p.G <= 64 || (p.G <= 128 && few)) && p.topk <= kMlaGMaxTopk &&
@@ -898,10 +897,18 @@ bool fwd_mla_supported(const Params& p) { return mla_supported(p); }
 
 // Whether p's kernel should walk ascending index rows: the persistent MLA
 // prefill, and the kernel for few heads when many queries run together over
-// more rows than an XCD's 4 MB L2 holds (2048 queries on 16384 keys, 16 / 32
-// heads: 0.53 / 0.67 -> 0.42 / 0.60 ms, the pass itself ~12 us; on 4096 keys
-// 115.1 -> 112.5 us, less than the pass), as for 128 heads below the
-// persistent kernel's 4096 queries (2048 on 16384 keys: 1082 -> 1045 us).
+// more rows than an XCD's 4 MB L2 holds, as for 128 heads below the persistent
+// kernel's 4096 queries.  us, rows as given -> with the pass (6 to 12 us of it):
+//   16 heads, 2048 queries, top-k 2048: on 8192 keys 432 -> 434, 16384 520 -> 444
+//   16 heads, 1024 queries, top-k  512: on 8192 keys 70.5 -> 76.1, 16384 81.6 -> 78.9
+//   32 heads, 2048 queries, top-k 2048: on 8192 keys 656 -> 639, 16384 679 -> 645
+//   32 heads, 1024 queries, top-k  512: on 8192 keys 104 -> 108, 16384 105 -> 109
+//   128 heads, 2048 queries, top-k 2048: on 8192 keys 1035 -> 1013, 16384 1061 -> 1030
+//   128 heads, 1024 queries, top-k 1024: on 8192 keys 289 -> 293, 16384 294 -> 298
+// so near 8192 keys, and with a short top-k, it gives back up to 8 %.  On 4096
+// keys the order alone gives at most 2 %, the pass more than that; 33 to 64
+// heads (bound by the matrix cores) lose with it at every size (2048 queries on
+// 16384 keys, top-k 2048: 1275 -> 1302).
 bool fwd_mfma_ascending(const Params& p) {
   if (p.num_splits != 1 || !idx_sort_supported(p)) return false;
   if (fwd_mfma_persistent(p)) return true;
@@ -932,8 +939,8 @@ bool fwd_mfma_supported(const Params& p) {
   return mla_supported(p) || fwd_mla_g_supported(p) || fwd_d128_supported(p);
 }
 
-// The MLA kernels hold all G heads of an item in one workgroup; the d = 128
-// kernel one head group of 16.
+// The 128-head MLA kernel holds all G heads of an item in one workgroup, the
+// kernel for few heads 16 or 32, the d = 128 kernel one head group of 16.
 int fwd_mfma_head_groups(const Params& p) {
   return mla_supported(p) ? 1 : fwd_mla_g_supported(p) ? fwd_mla_g_groups(p) : fwd_d128_head_groups(p);
 }

@@ -10,7 +10,7 @@
 // so the kernel is built around the gather:
 //  * one workgroup of 4 waves per (batch, query, kv head[, split]) and all its
 //    heads (up to 32, NG groups of 16, the MFMA's N; more take a workgroup per
-//    32, on one XCD); 32-key tiles of whole 1152-byte
+//    32); 32-key tiles of whole 1152-byte
 //    rows straight into LDS (RowGather), double buffered, 78 KB, so that two
 //    workgroups share a CU and one's products cover the other's waits;
 //  * S^T = K Q^T is divided over the waves by key half and, with 16 heads, by
@@ -26,11 +26,11 @@
 // float64 result, over prefills and decodes of 16 to 64 heads: 1.8e-4 to 3.0e-4
 // (scalar kernel 1.7e-4 to 5.5e-4; with two terms 1.7e-3 to 2.3e-3, at 450
 // against 485 us for 2048 queries of 16 heads, 1110 against 1290 us of 64).
-// Bound: the gather with 16 heads (9.1 TB/s from the Infinity Cache of the
-// 11 TB/s that whole rows reach there; 11.4 TB/s on ascending index rows, part
-// of it from L2), the matrix cores with 64.  2048 queries on 16384 keys, top-k
-// 2048, 16 heads: 0.52 ms, 0.43 ms on ascending rows, 64.5 ms on the scalar
-// kernel (one workgroup per query and head); 64 heads 1.18 ms.
+// Bound: with 16 heads the gather (4.8 GB in 0.44 ms, 11 TB/s, three quarters of
+// it from L2 on ascending index rows, the rest from the Infinity Cache) and the
+// serial chain of a tile, the matrix cores with 64.  2048 queries on 16384 keys,
+// top-k 2048, 16 heads: 0.52 ms, 0.44 ms on ascending rows, 64.5 ms on the
+// scalar kernel (one workgroup per query and head); 64 heads 1.28 ms.
 // Up to 4 queries of 65 to 128 heads (a few sequences' decode step) take it
 // too, 16 heads per workgroup: the 128-head kernel loads all 147 KB of Q in
 // every split before its first product.
@@ -94,7 +94,8 @@ __global__ __launch_bounds__(256, 2) void fwd_mla_g_kernel(Params p) {
 
   // ---- work item: its splits and head groups on one XCD (workgroup id % 8:
   // they share its Q or its rows), unsplit items in runs of 32 consecutive
-  // queries on one XCD (shared keys meet in its L2) ---------------------------
+  // queries on one XCD (shared keys meet in its L2); the last items, fewer than
+  // 8, spread theirs over the XCDs (all of a small decode step: more CUs) ------
   const int64_t nitems = (int64_t)p.B * p.Sq * p.Hkv;
   const int nhg = (p.G + 16 * NG - 1) / (16 * NG), nsub = p.num_splits * nhg;
   const int runs = p.num_splits == 1 ? (int)(nitems / 256 * 256) : 0;  // items placed in runs

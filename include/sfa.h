@@ -215,8 +215,8 @@ SFA_API int sfa_fwd(const sfa_fwd_args* a, void* workspace, size_t workspace_byt
  * buffer of SFA_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds
  * until the process ends; a plan that needs more returns SFA_E_WORKSPACE
  * before any device work, with two exceptions.  The kernel for up to 64 heads
- * (and for up to 4 queries of up to 128) on MLA rows is split no further than
- * its fp32 partials fit.  The prefill's sorted index rows: when they do not
+ * (and for up to 4 queries of up to 128 with 16384 index slots in all) on MLA
+ * rows is split no further than its fp32 partials fit.  The prefill's sorted index rows: when they do not
  * fit, the rows are walked in their own order (the result then equals
  * sfa_fwd's with SFA_FWD_IDX_SORTED set; bitwise equal to sfa_fwd whenever the
  * sorted rows fit or the rows are already ascending).  `stream` must belong to

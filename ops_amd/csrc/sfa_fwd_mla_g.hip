@@ -31,8 +31,8 @@
 // serial chain of a tile, the matrix cores with 64.  2048 queries on 16384 keys,
 // top-k 2048, 16 heads: 0.52 ms, 0.44 ms on ascending rows, 64.5 ms on the
 // scalar kernel (one workgroup per query and head); 64 heads 1.28 ms.
-// Up to 4 queries of 65 to 128 heads (a few sequences' decode step) take it
-// too, 16 heads per workgroup: the 128-head kernel loads all 147 KB of Q in
+// Up to 4 queries of 65 to 128 heads with 16384 slots in all (a few sequences'
+// decode step) take it too, 16 heads per workgroup: the 128-head kernel loads all 147 KB of Q in
 // every split before its first product.
 
 #include "sfa_common.h"
